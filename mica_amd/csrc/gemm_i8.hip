@@ -773,6 +773,12 @@ int mm_i8_run(const int8_t *A, int lda, const int8_t *B, int ldb, const float *s
     int grid = (int)tiles;
     int dev = 0;
     const int cus = hipGetDevice(&dev) == hipSuccess ? cu_count(dev) : 0;
+    // Few rows: one round of small tiles (gemm_i8_thin.hip; same bits as every other schedule)
+    if (cus > 0 && (out_dtype == MICA_BF16 || out_dtype == MICA_FP16) && (long long)(M + kTile) * lda < (1ll << 31) &&
+        (long long)(N + kTile) * ldb < (1ll << 31)) {
+        int rc = 0;
+        if (thin_launch(p, epilogue, out_dtype, cus, bias != nullptr, residual != nullptr, st, &rc)) return rc;
+    }
     // Few tiles and a long K (a short request's down projection, e.g. 128 x 2560 x 9728: 16 tiles of
     // 128 x 160 on 256 CUs): with a workspace, one round of 128-row tiles split along K into `parts`
     // pieces whose int32 partial sums each tile's last part adds (agpr_split_launch; same bits as every

@@ -1,4 +1,5 @@
-// Pieces shared by the two W8A8 GEMM kernels (gemm_i8.hip, gemm_i8_wide.hip): the launch parameters,
+// Pieces shared by the W8A8 GEMM kernels (gemm_i8.hip, gemm_i8_wide.hip, gemm_i8_agpr.hip,
+// gemm_i8_thin.hip): the launch parameters,
 // the XCD-aware tile order, wait helpers and the epilogue's 4-value loads and stores.
 #pragma once
 
@@ -148,6 +149,11 @@ int agpr_silu_small_launch(const GemmParams &p, int grid, hipStream_t st);
 int agpr_split_tile_n(int epilogue);
 long long agpr_split_slot_bytes(int epilogue);
 int agpr_split_launch(const GemmParams &p, int epilogue, int out_dtype, bool has_bias, bool has_res, hipStream_t st);
+
+// one round of small tiles for few rows (gemm_i8_thin.hip): 16-bit outputs, operands addressable one 256-row
+// tile past their last row.  False when no tile suits the launch, else *rc is the launch's result.
+bool thin_launch(const GemmParams &p, int epilogue, int out_dtype, int cus, bool has_bias, bool has_res, hipStream_t st,
+                 int *rc);
 
 }  // namespace mica_gemm
 

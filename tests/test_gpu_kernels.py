@@ -606,6 +606,53 @@ def test_gemm_small_m_split_bit_exact(gpu, m, n, k, epi):
         assert np.array_equal(got.view(np.uint16), plain.view(np.uint16)), f"split != unsplit (call {rep})"
 
 
+@pytest.mark.parametrize("m,n,k,epi", [
+    (1, 2560, 9728, "residual"),        # 16 x 16 tiles, K split over 4 waves, 15 of 16 rows past the end
+    (17, 2568, 512, "bias"),            # 16 x 32, one slab, both edges ragged
+    (16, 10240, 2560, "none"),          # 16 x 64
+    (33, 2500, 1024, "bias_fp16"),      # 32 x 32, N a multiple of 4 only
+    (100, 2562, 4096, "residual"),      # 64 x 32, element stores (N even only)
+    (33, 9001, 512, "bias_residual"),   # 32 x 128, odd N
+    (384, 2560, 9728, "residual"),      # 64 x 64, K split over 2 waves, the most rows and bytes per tile
+    (200, 10240, 2560, "none"),         # 128 x 128
+    (127, 10240, 2560, "bias"),         # 128 x 64
+    (192, 10240, 2560, "none"),         # 64 x 128
+    (48, 300, 128, "none"),             # one slab of 128 bytes: the tiles that do not split K
+    (5, 32, 384, "none"),               # three slabs, N below a tile
+    (8, 19456, 2560, "silu_mul"),       # 32 x 128: 64 gate and 64 up rows
+    (64, 19456, 2560, "silu_mul"),      # 64 x 128
+    (128, 19456, 2560, "silu_mul"),     # 128 x 128
+    (20, 640, 512, "silu_mul"),         # 16 x 32: 16 gate and 16 up rows
+    (33, 3200, 1024, "silu_mul"),       # 32 x 32, ragged rows
+    (300, 4224, 256, "silu_mul"),       # 64 x 64, one slab, a last tile past the output
+])
+def test_gemm_few_rows_bit_exact(gpu, m, n, k, epi):
+    """Up to 384 rows: one round of small tiles whose waves split K (int32 sums, exact in any order).  Bit-exact
+    with the oracle; the SiLU within the one-ulp bound of its own test."""
+    note(f"gemm few rows m={m} n={n} k={k} epi={epi}")
+    rng = np.random.default_rng(m * 5 + n + k)
+    A, B, sa, sb = _rand_gemm(rng, m, n, k)
+    tA, tB, tsa, tsb = (torch.from_numpy(v).cuda() for v in (A, B, sa, sb))
+    if epi == "silu_mul":
+        n2 = n // 2
+        grp, sgr = B.reshape(n // 128, 2, 64, k), sb.reshape(n // 128, 2, 64)
+        gv, uv = (O.epilogue(O.int_gemm(A, grp[:, i].reshape(n2, k)), sa, sgr[:, i].reshape(n2)) for i in (0, 1))
+        assert_within_one_ulp(bits_of(int8_kernels.mm_i8(tA, tsa, tB, tsb, epilogue="silu_mul")), O.silu_mul(gv, uv))
+        return
+    bias = rng.uniform(-1, 1, n).astype(np.float32) if "bias" in epi else None
+    tb = None if bias is None else torch.from_numpy(bias).cuda()
+    acc = O.int_gemm(A, B)
+    if epi == "bias_fp16":
+        y = int8_kernels.mm_i8(tA, tsa, tB, tsb, tb, out_dtype=torch.float16)
+        assert_equal_diag(y.cpu().numpy(), O.epilogue(acc, sa, sb, bias, "fp16"), "fp16")
+        return
+    ref, res = O.epilogue(acc, sa, sb, bias), None
+    if "residual" in epi:
+        rb = act_bits(rng, (m, n), outliers=0)
+        res, ref = to_gpu_bf16(rb), O.f32_to_bf16(O.bf16_to_f32(ref) + O.bf16_to_f32(rb))
+    assert_equal_diag(bits_of(int8_kernels.mm_i8(tA, tsa, tB, tsb, tb, residual=res)), ref, "bf16")
+
+
 @pytest.mark.parametrize("m,n,k", [(32768, 6144, 2560), (32768, 2560, 4096)])
 def test_gemm_config3_long_context_sampled_rows(gpu, m, n, k):
     """Config 3 (T = 32768 packed prefill): QKV 2560 -> 6144 and O 4096 -> 2560, checked exactly on a
