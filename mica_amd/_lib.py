@@ -1,4 +1,5 @@
-"""ctypes binding of libmica_amd.so, the C ABI declared in include/mica_amd.h.
+"""ctypes binding of libmica_amd.so, the C ABI declared in include/mica_amd.h, and the loader of the native
+launch path over it (binding/native.cpp, _native.so).
 
 The library is loaded after torch, so it binds to the HIP runtime torch already loaded (same soname)
 and the stream handles torch hands out are valid in it.  A missing library is an error, never a
@@ -7,6 +8,8 @@ silent fallback: build it with ``python -m mica_amd.build``.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from pathlib import Path
@@ -69,6 +72,24 @@ SIGNATURES = {
     "mica_gdn_gate": (_I, [_P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _P]),
 }
 
+# functions of libmica_amd.so that the native launch path calls
+NATIVE_FNS = ("mica_act_quant", "mica_mm_i8", "mica_rmsnorm_quant", "mica_rmsnorm_quant_multi",
+              "mica_attention_prefix_workspace_bytes", "mica_attention_fwd", "mica_attention_fwd_prefix",
+              "mica_causal_conv1d", "mica_gdn_chunk", "mica_gdn_workspace_bytes", "mica_gdn_gate",
+              "mica_gated_rmsnorm_quant")
+
+
+class _NotLoaded:
+    """Stands for the native launch path until load(): every function declines the call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+# binding/native.cpp's functions: each launches a plain call and returns its result, or None for a call that the
+# Python path has to serve or refuse, or the negative error of a failed launch (int)
+FAST = _NotLoaded()
+
 _LIB = None
 _LOCK = threading.Lock()
 
@@ -78,9 +99,20 @@ def lib_path() -> Path:
     return (Path(d) if d else Path(__file__).resolve().parent) / LIB_NAME
 
 
+def _load_native(lib):
+    path = Path(__file__).resolve().parent / "_native.so"
+    if not path.is_file():
+        raise RuntimeError(f"{path} is not built; run `python -m mica_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("mica_amd._native", str(path))
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("mica_amd._native", loader))
+    loader.exec_module(mod)
+    mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in NATIVE_FNS})
+    return mod
+
+
 def load():
     """Load (once) and return the ctypes library; raises RuntimeError if it is not built."""
-    global _LIB
+    global _LIB, FAST
     if _LIB is not None:
         return _LIB
     with _LOCK:
@@ -94,6 +126,7 @@ def load():
             for name, (res, args) in SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.restype, fn.argtypes = res, args
+            FAST = _load_native(lib)
             _LIB = lib
     return _LIB
 

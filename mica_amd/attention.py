@@ -14,7 +14,7 @@ import math
 import torch
 
 from . import _lib
-from .int8_kernels import _aligned, _gpu_ok, _launched, _on, _stream
+from .int8_kernels import _aligned, _gpu_ok, _launched, _native, _on, _stream
 
 HEAD_DIM = 256
 GROUP = 4
@@ -60,6 +60,12 @@ def attention_fwd(q, k, v, q_layout: str, scale: float | None = None, key_splits
     bf16((x rstd) (offset + w)), a weight of None skipping that side.  k is treated in place, exactly as
     ``fused_kernels.rope_inplace`` / ``head_norm_rope`` treat it; q as the kernel loads it, unchanged in
     memory.  The result equals those passes over q and k followed by the plain call, bit for bit."""
+    if kv_len is None and rope is None and head_norm is None and key_splits == 1 and q_layout in ("bshd", "bhsd"):
+        kp, vp = prefix if prefix is not None else (None, None)
+        r = _lib.FAST.attention(q, k, v, q_layout == "bshd",
+                                1.0 / math.sqrt(HEAD_DIM) if scale is None else float(scale), kp, vp)
+        if r is not None:
+            return _native(r, "mica_attention_fwd")
     for t in (q, k, v):
         if not t.is_cuda:
             raise ValueError("mica_amd attention runs on the GPU only (got a CPU tensor)")

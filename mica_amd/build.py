@@ -1,4 +1,5 @@
-"""Build libmica_amd.so in-tree: every source under mica_amd/csrc compiled for gfx950 with hipcc.
+"""Build libmica_amd.so in-tree: every source under mica_amd/csrc compiled for gfx950 with hipcc; and _native.so,
+the host-side launch path (mica_amd/binding), with g++ against torch's headers.
 
     python -m mica_amd.build [--jobs N]
 
@@ -19,6 +20,8 @@ from pathlib import Path
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT = PKG / "libmica_amd.so"
+BINDING = PKG / "binding" / "native.cpp"
+NATIVE = PKG / "_native.so"
 OBJ = PKG / "_build"
 ARCH = "gfx950"
 
@@ -55,13 +58,41 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _run(cmd, what):
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+
+
+def build_native() -> Path:
+    """Compile the launch path into _native.so (a CPython module; it calls libmica_amd.so through the addresses
+    _lib.load() gives it, so the two are linked only to torch and Python)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension as ext
+
+    rocm = Path(hipcc()).resolve().parent.parent
+    libs = ext.library_paths()
+    tmp = NATIVE.with_suffix(".so.tmp")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM=1",
+          "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *[f"-I{p}" for p in (*ext.include_paths(), rocm / "include", sysconfig.get_paths()["include"])],
+          str(BINDING), "-o", str(tmp), *[f"-L{p}" for p in libs], *[f"-Wl,-rpath,{p}" for p in libs],
+          "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"], "g++ for native.cpp")
+    os.replace(tmp, NATIVE)
+    return NATIVE
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> Path:
-    """Compile every source (always; never trusts an existing library) and link libmica_amd.so."""
+    """Compile every source (always; never trusts an existing library), link libmica_amd.so and _native.so."""
     OBJ.mkdir(exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), os.cpu_count() or 4)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        native = ex.submit(build_native)
         objs = list(ex.map(_compile, srcs))
+        native.result()
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)

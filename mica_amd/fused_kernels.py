@@ -17,7 +17,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .int8_kernels import DT, ROUNDING, _aligned, _gpu_ok, _launched, _miss, _on, _stream
+from .int8_kernels import DT, ROUNDING, _aligned, _gpu_ok, _launched, _miss, _native, _on, _stream
 
 NORM_DT = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16}
 
@@ -39,6 +39,14 @@ def _check_row_input(x, weight, residual):
 
 
 def _launch_norm(x, weight, eps, residual, offset, inv_smooth, want_q, want_y, rounding):
+    r = _lib.FAST.norm(x, weight, float(eps), residual, float(offset), inv_smooth, want_q, want_y,
+                       ROUNDING.get(rounding, -1))
+    if r is not None:
+        return _native(r, "mica_rmsnorm_quant")
+    _check_row_input(x, weight, residual)
+    if inv_smooth is not None and (inv_smooth.dtype != torch.float32 or inv_smooth.numel() != x.shape[-1]
+                                   or not inv_smooth.is_contiguous() or inv_smooth.device != x.device):
+        raise ValueError("inv_smooth must be a contiguous fp32 [K] tensor on x's device")
     K = x.shape[-1]
     flat = x.reshape(-1, K)
     if flat.stride(0) != K:
@@ -81,6 +89,10 @@ def rms_norm_quant_multi(x, weight, eps, inv_smooths, residual=None, offset=1.0,
     Returns a list of (q_i, s_i), each equal to ``rms_norm_quant(x, weight, eps, inv_smooths[i], ...)``,
     plus the summed input v when ``residual`` is given: ([(q, s), ...], v).
     """
+    r = _lib.FAST.norm_multi(x, weight, float(eps), inv_smooths, residual, float(offset), ROUNDING.get(rounding, -1))
+    if r is not None:
+        out, summed = _native(r, "mica_rmsnorm_quant_multi")
+        return out if residual is None else (out, summed)
     _check_row_input(x, weight, residual)
     K = x.shape[-1]
     n = len(inv_smooths)
@@ -138,7 +150,6 @@ def rms_norm(x, weight, eps, residual=None, offset=1.0):
     (fused_kernels.py:51-56), this raises ValueError naming the device, so a CPU caller has to norm
     its rows itself.
     """
-    _check_row_input(x, weight, residual)
     _, _, y, summed = _launch_norm(x, weight, eps, residual, offset, None, False, True, "even")
     return y if residual is None else (y, summed)
 
@@ -151,11 +162,6 @@ def rms_norm_quant(x, weight, eps, inv_smooth=None, residual=None, offset=1.0, r
     and s fp32 [M] over the flattened rows.  Returns (q, s), plus the bf16 normed rows when
     ``return_normed``, plus the summed input v when ``residual`` is given: (q, s[, y][, v]).
     """
-    _check_row_input(x, weight, residual)
-    K = x.shape[-1]
-    if inv_smooth is not None and (inv_smooth.dtype != torch.float32 or inv_smooth.numel() != K
-                                   or not inv_smooth.is_contiguous() or inv_smooth.device != x.device):
-        raise ValueError("inv_smooth must be a contiguous fp32 [K] tensor on x's device")
     q, s, y, summed = _launch_norm(x, weight, eps, residual, offset, inv_smooth, True, return_normed, rounding)
     out = (q, s)
     if return_normed:

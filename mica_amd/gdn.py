@@ -22,7 +22,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .int8_kernels import _aligned, _gpu_ok, _launched, _on, _stream
+from .int8_kernels import _aligned, _gpu_ok, _launched, _native, _on, _stream
 
 HEAD_DIM = 128
 CHUNK = 64
@@ -60,6 +60,12 @@ def causal_conv1d_fn(x, weight, bias=None, seq_idx=None, initial_states=None, re
     SiLU when activation is 'silu' / 'swish'.  Returns y [B, C, T] bf16 (a channel-last view), and
     the final states [B, C, W - 1] when return_final_states.  l2norm_heads > 0 also divides each of
     the first l2norm_heads 128-channel groups of every token by its l2 norm (+ eps)."""
+    if seq_idx is None and final_states_out is None and activation in (None, "silu", "swish"):
+        r = _lib.FAST.conv(x, weight, bias, initial_states, return_final_states, activation is not None,
+                           int(l2norm_heads), float(eps))
+        if r is not None:
+            r = _native(r, "mica_causal_conv1d")
+            return r if return_final_states else r[0]
     if seq_idx is not None:
         raise ValueError("seq_idx is not supported")
     if activation not in (None, "silu", "swish"):
@@ -139,6 +145,11 @@ def chunk_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None, out
     Returns (o bf16 [B, T, HV, 128], final_state fp32 [B, HV, 128, 128] or None)."""
     if cu_seqlens is not None or head_first:
         raise ValueError("cu_seqlens / head_first layouts are not supported")
+    if not use_qk_l2norm_in_kernel:
+        r = _lib.FAST.gdn_chunk(q, k, v, g, beta, HEAD_DIM ** -0.5 if scale is None else float(scale), initial_state,
+                                output_final_state)
+        if r is not None:
+            return _native(r, "mica_gdn_chunk")
     dev = _need_gpu(q, k, v, g, beta, initial_state)
     if use_qk_l2norm_in_kernel:
         q, k = l2norm_heads(q), l2norm_heads(k)
@@ -181,6 +192,9 @@ def gdn_gate(a, b, A_log, dt_bias):
     g = -exp(A_log) * softplus(a + dt_bias) (fp32) and beta = sigmoid(b) (bf16), per token and value
     head.  a, b: bf16 [..., HV] (rows may be strided); A_log, dt_bias: [HV].  Returns (g, beta) shaped
     like a."""
+    r = _lib.FAST.gdn_gate(a, b, A_log, dt_bias)
+    if r is not None:
+        return _native(r, "mica_gdn_gate")
     dev = _need_gpu(a, b, A_log, dt_bias)
     HV = a.shape[-1]
     af, bf = a.reshape(-1, HV), b.reshape(-1, HV)
@@ -204,6 +218,10 @@ def gdn_gate(a, b, A_log, dt_bias):
 def gated_rmsnorm_quant(x, z, weight, eps: float = 1e-6, want_y: bool = False):
     """attn.norm(x, z) over 128-wide heads, then per-token INT8 (half-even) of the [.., HV * 128] row.
     Returns (q int8 [M, N], s fp32 [M]) or, with want_y, (q, s, y bf16 [M, N])."""
+    r = _lib.FAST.gated_norm(x, z, weight, float(eps), want_y)
+    if r is not None:
+        r = _native(r, "mica_gated_rmsnorm_quant")
+        return r if want_y else r[:2]
     dev = _need_gpu(x, z, weight)
     N = x.shape[-1]
     xf = x.reshape(-1, N)
@@ -266,10 +284,7 @@ class GDNLayer(torch.nn.Module):
                                 initial_states=init_conv, return_final_states=keep, l2norm_heads=2 * self.hk)
         conv, conv_state = conv if keep else (conv, None)
         x = conv.transpose(1, 2)                            # [B, T, C] (contiguous memory)
-        kd = self.hk * HEAD_DIM
-        q = x[..., :kd].unflatten(-1, (self.hk, HEAD_DIM))
-        k = x[..., kd:2 * kd].unflatten(-1, (self.hk, HEAD_DIM))
-        v = x[..., 2 * kd:].unflatten(-1, (self.hv, HEAD_DIM))
+        q, k, v = x.view(batch, T, -1, HEAD_DIM).split((self.hk, self.hk, self.hv), dim=2)
         g, beta = gdn_gate(a, b, self.A_log, self.dt_bias)
         o, rec = chunk_gated_delta_rule(q, k, v, g.view(batch, T, self.hv), beta.view(batch, T, self.hv),
                                         initial_state=None if initial is None else initial[1],

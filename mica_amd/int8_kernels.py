@@ -56,6 +56,14 @@ def _launched():
         STATS["launch"] += 1
 
 
+def _native(r, name):
+    """The result of a native launch (_lib.FAST; not None): counted, an error code raised."""
+    if type(r) is int:
+        _lib.check(r, name)
+    _launched()
+    return r
+
+
 ENV_DIR = "MICA_W8A8_AOT_DIR"   # int8_kernels.py:10
 
 
@@ -87,6 +95,8 @@ def _gfx(dev) -> int:
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     if idx not in _ARCH:
         _ARCH[idx] = _lib.device_info(idx)["gfx_arch"]
+        if _ARCH[idx] == 950:
+            _lib.FAST.device_ok(idx)
     return _ARCH[idx]
 
 
@@ -178,6 +188,7 @@ def gemm_workspace(dev, stream=None):
                 ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
                 _WORKSPACE[key] = ws
                 _WS_PTR[key] = (ws.data_ptr(), ws.numel())
+                _lib.FAST.workspace(*key, *_WS_PTR[key])
     return ws.data_ptr(), ws.numel()
 
 
@@ -208,6 +219,9 @@ def auto_split(dev):
 
 def act_quant(x, inv_smooth=None, rounding="even"):
     """Per-token INT8 quantization of a 2-D activation (int8_kernels.py:325-353)."""
+    r = _lib.FAST.act_quant(x, inv_smooth, ROUNDING.get(rounding, -1))
+    if r is not None:
+        return _native(r, "mica_act_quant")
     if x.dim() != 2 or x.device.type != "cuda" or x.dtype not in DT:
         return _miss("act_input")
     m, k = x.shape
@@ -250,6 +264,11 @@ def mm_i8(qx, sx, qw, sw, bias=None, out_dtype=torch.bfloat16, residual=None, ep
     a second launch, because each row's scale needs the absmax of the whole row, which spans every
     column tile of the GEMM.
     """
+    out = _lib.FAST.mm_i8(qx, sx, qw, sw, bias, DT.get(out_dtype, -1), residual, EPILOGUE.get(epilogue, -1),
+                          bool(split) and (split != "auto" or SPLIT["auto"]))
+    if out is not None:
+        _native(out, "mica_mm_i8")
+        return act_quant(out) if requant else out
     if qx.dim() != 2 or qw.dim() != 2 or qx.dtype != torch.int8 or qw.dtype != torch.int8 or out_dtype not in DT:
         return _miss("mm_input")
     m, k = qx.shape
