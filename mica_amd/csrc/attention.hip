@@ -57,12 +57,19 @@ constexpr int kFaThreads = 64 * kFaWaves;
 constexpr int kKBytes = kBK * kD * 2;    // 16 KB: 32 key rows x 512 B
 constexpr int kVBytes = kD * kBK * 2;    // 16 KB: 256 dim rows x 64 B
 constexpr int kStage = kKBytes + kVBytes;
-#ifndef MICA_FA_OCC
-#define MICA_FA_OCC 2
-#endif
 constexpr int kNSt = 2;                  // LDS stages: tile j + 1 in flight while tile j is read
-constexpr int kFaSmem = kNSt * kStage;   // also the output staging (4 waves x 32 x 512 B) after the loop
+constexpr int kPSt = 4;                  // the pipelined schedule's: one read, one landed, two in flight
+// LDS: the operand stages, after the loop the output staging (4 waves x 32 x 512 B)
+template <bool PIPE>
+constexpr int kFaSmem = (PIPE ? kPSt : kNSt) * kStage;
 constexpr int kMaxKeySplits = 64;
+// The pipelined schedule serves grids of at most kPipeBlocks workgroups (2 per CU) whose blocks walk at least
+// kPipeKeys keys: there a wave's chain of tiles is what takes the time.  Measured on MI355X (us, two workgroups per
+// CU / pipelined): 1 x 2048 78.2 / 73.5, 1 x 3000 118.1 / 105.9, 4 x 700 42.7 / 40.1, 8 x 240 after 6912 keys 267 / 248,
+// 8 x 64 after 6912 220 / 193; shorter or fuller grids lose by its longer prologue and its one workgroup per CU:
+// 8 x 256 21.9 / 23.7, 8 x 512 39.0 / 45.8, 1 x 256 19.4 / 20.7, 4 x 1500 (752 workgroups) 95.8 / 114.7.
+constexpr int kPipeBlocks = 512;
+constexpr int kPipeKeys = 640;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -243,9 +250,11 @@ __global__ __launch_bounds__(256) void v_transpose_kernel(FaParams p) {
     }
 }
 
-template <bool SPLIT>
-__global__ __launch_bounds__(kFaThreads, MICA_FA_OCC) void fa_fwd_kernel(FaParams p) {
-    __shared__ __attribute__((aligned(1024))) int8_t smem[kFaSmem];
+// PIPE: the schedule of small grids over long keys (kPipeBlocks), one workgroup per CU and one wave per SIMD;
+// otherwise two workgroups per CU, whose waves fill each other's gaps.  Same bits.
+template <bool SPLIT, bool PIPE>
+__global__ __launch_bounds__(kFaThreads, PIPE ? 1 : 2) void fa_fwd_kernel(FaParams p) {
+    __shared__ __attribute__((aligned(1024))) int8_t smem[kFaSmem<PIPE>];
     // grid (HK, B, ntiles_q [x nsplit]): every (sequence, head) pair's longest query blocks are
     // dispatched first
     const int qblk = p.ntiles_q - 1 - (SPLIT ? (int)blockIdx.z / p.nsplit : (int)blockIdx.z);
@@ -301,6 +310,43 @@ __global__ __launch_bounds__(kFaThreads, MICA_FA_OCC) void fa_fwd_kernel(FaParam
         for (int i = 0; i < 4; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rvs, (lds_void *)(ks + kKBytes + (wave * 4 + i) * 1024), 16,
                                                      ln * 16, jj * kVBytes + (wave * 4 + i) * 1024, 0, 0);
+    };
+
+    // The pipelined schedule's DMA, an instruction range at a time (addresses and sizes as scalars; a tile's resource is
+    // built where it is used).
+    const uint64_t ka = (uint64_t)(p.k + b * p.sbk + hk * p.shk), va = (uint64_t)(p.vt + ((long long)(b * p.HK + hk) * ntn) * kD * kBK);
+    const uint64_t kpa = (uint64_t)(ntp ? p.kp + hk * p.shkp : p.k), vpa = (uint64_t)(ntp ? p.vtp + ((long long)hk * ntp) * kD * kBK : p.vt);
+    const int kn = (int)((long long)(p.Sk - pk) * p.ldk * 2), vn = ntn * kVBytes, kpn = (int)((long long)pk * p.ldkp * 2), vpn = ntp * kVBytes;
+    int8_t *const sm = smem;
+    int ko_own[4], ko_diff[4]; // a prefix tile's offset less an own tile's
+    const int tile_own = (int)(kBK * p.ldk * 2), tile_pre = (int)(kBK * p.ldkp * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = (wave * 4 + i) * 2 + hi;
+        ko_own[i] = (int)(row * p.ldk * 2) + ((l32 ^ row) << 4);
+        ko_diff[i] = (int)(row * (p.ldkp - p.ldk) * 2);
+    }
+    // Tiles outside first .. last_own load from a zero-sized buffer, zeros into a stage, so that every tile step issues
+    // the same number of vector memory operations (which its vmcnt waits count).
+    auto dma_k = [=](int j, int st, int i0, int i1) {
+        const bool pre = j < ntp;  // the tile's segment: the shared prefix or this sequence's own keys
+        const uint64_t at = pre ? kpa + 0 : ka + 0;
+        const int n = j > last_own ? 0 : pre ? kpn + 0 : kn + 0, tile_off = pre ? j * tile_pre : (j - ntp) * tile_own;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)at, 0, n, kBufferFlags);
+#pragma unroll
+        for (int i = i0; i < i1; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(sm + st * kKBytes + (wave * 4 + i) * 1024), 16,
+                                                     ko_own[i] + (pre ? ko_diff[i] : 0) + tile_off, 0, 0, 0);
+    };
+    auto dma_v = [=](int j, int st, int i0, int i1) {
+        const bool pre = j < ntp;
+        const uint64_t at = pre ? vpa + 0 : va + 0;
+        const int n = j > last_own || j < first ? 0 : pre ? vpn + 0 : vn + 0, jj = pre ? j : j - ntp;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)at, 0, n, kBufferFlags);
+#pragma unroll
+        for (int i = i0; i < i1; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(sm + kPSt * kKBytes + st * kVBytes + (wave * 4 + i) * 1024),
+                                                     16, lane * 16, jj * kVBytes + (wave * 4 + i) * 1024, 0, 0);
     };
 
     // Q fragments (B operand of S^T): lane holds query q0 + l % 32, dims 16 s + 8 (l / 32) .. + 7
@@ -377,6 +423,7 @@ __global__ __launch_bounds__(kFaThreads, MICA_FA_OCC) void fa_fwd_kernel(FaParam
     int vfoff[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) vfoff[s] = l32 * (kBK * 2) + (((2 * s + hi) ^ vt_swz(l32)) << 4);
+    if constexpr (!PIPE) {
     // tile j in stage (j - first) % 2, the other stage receiving tile j + 1
     if (first <= last_own) dma_tile(first, 0);
     for (int j = first; j <= last_own; ++j) {
@@ -461,6 +508,177 @@ __global__ __launch_bounds__(kFaThreads, MICA_FA_OCC) void fa_fwd_kernel(FaParam
             __builtin_amdgcn_sched_barrier(0);
             O[m & 7] = mfma_bf16(a, pb[m >> 3], O[m & 7]);
         }
+    }
+    } else {
+    constexpr int kPf = 4; // operand fragments are read this many steps (two MFMAs each) ahead
+    auto kfrag = [&](int st, int s) {
+        return __builtin_bit_cast(bf16x8, *(const u32x4 *)(smem + st * kKBytes + kfoff + (((2 * s + hi) ^ l32) * 16)));
+    };
+    // V^T operand of step m = 8 s + dt: every dim tile's step 0, then its step 1
+    auto vfrag = [&](int st, int m) {
+        return __builtin_bit_cast(bf16x8, *(const u32x4 *)(smem + kPSt * kKBytes + st * kVBytes + vfoff[m >> 3] +
+                                                           (m & 7) * 32 * (kBK * 2)));
+    };
+    // masked scores of tile j where it does not lie wholly at or below the block's diagonal
+    auto mask = [&](int j, f32x16 &sc) {
+        if (j * kBK + kBK - 1 > off + q0) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                sc[r] = j * kBK + 8 * (r >> 2) + 4 * hi + (r & 3) <= query ? sc[r] : -__builtin_inff();
+        }
+    };
+    // K of tile t lives in stage t % 4, V^T of tile t likewise (t counted from the first tile)
+    f32x16 sc = {};
+    bf16x8 kf[kPf], vf[kPf];   // the fragments read ahead: K of tile j + 1, V^T of tile j - 1
+    if (first <= last_own) {
+        dma_k(first, 0, 0, 4);
+        dma_k(first + 1, 1, 0, 4);
+        dma_v(first - 1, 3, 0, 4);   // zeros: the first step's product adds nothing
+        dma_k(first + 2, 2, 0, 4);
+        dma_v(first, 0, 0, 4);
+        dma_k(first + 3, 3, 0, 4);
+        dma_v(first + 1, 1, 0, 4);
+        fa_wait_vmcnt<16>();   // K of the first two tiles, the zeros
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kPf; ++i) kf[i] = kfrag(0, i);
+#pragma unroll
+        for (int s = 0; s < kD / 16; ++s) {
+            const bf16x8 a = kf[s % kPf];
+            kf[s % kPf] = s + kPf < kD / 16 ? kfrag(0, s + kPf) : kfrag(1, s + kPf - kD / 16);
+            __builtin_amdgcn_sched_barrier(0);
+            sc = mfma_bf16(a, qf[s], sc);
+        }
+#pragma unroll
+        for (int i = 0; i < kPf; ++i) vf[i] = vfrag(3, i);
+    }
+    // Tile step j: the 16 MFMAs of S(j + 1) = K Q^T and the 16 of O += V P of tile j - 1 in turn, with the softmax of
+    // tile j beside them (maximum, reference, exponentials, packing: all VALU, no branch).  The one wave of a SIMD so
+    // keeps its MFMA pipe fed, and no MFMA waits for the one before it: consecutive accumulations of the S chain
+    // are two slots apart (two in a row measured 14 % slower: 8 x 64 after 6912 keys 193 -> 224 us).
+    bf16x8 pv[2] = {};       // P of the tile before, zero at first
+    float pe[16];
+    uint32_t pw[8];
+    // p = 2^(scale s - m) of score r, the scaling fused into the exponent's argument; pairs summed and packed
+    // (the empty asm keeps each value in its step: the compiler otherwise sinks them past the last MFMA)
+    auto prob = [&](int r) {
+        pe[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], p.scale_log2, -m_used));
+        __asm__ volatile("" : "+v"(pe[r]));
+    };
+    auto pair = [&](int i) {
+        lsum += pe[2 * i] + pe[2 * i + 1];
+        pw[i] = pack_bf16x2(pe[2 * i], pe[2 * i + 1]);
+        __asm__ volatile("" : "+v"(pw[i]), "+v"(lsum));
+    };
+    for (int j = first; j < last_own; ++j) {
+        const int t = j - first, st = t % kPSt, sk = (t + 1) % kPSt, sk2 = (t + 2) % kPSt, sv = (t + 3) % kPSt;
+        // this wave's DMA of K(j + 2) and V(j) landed (those of the last step, 8, may still be out); after the barrier
+        // every wave's has, and nobody reads K(j) or V(j - 2) any more: K(j + 4) and V(j + 2) go there.  K(j + 1) and
+        // V(j - 1) were there a barrier earlier, so their first fragments are in registers already.
+        fa_wait_vmcnt<8>();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        mask(j, sc);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 sn = {};
+        float mx = -__builtin_inff(), alpha = 1.0f;
+        bool grow = false;
+#pragma unroll
+        for (int s = 0; s < kD / 16; ++s) {
+            const bf16x8 a = kf[s % kPf], b2 = vf[s % kPf];
+            if (s + kPf < kD / 16) {
+                kf[s % kPf] = kfrag(sk, s + kPf);
+                vf[s % kPf] = vfrag(sv, s + kPf);
+            } else { // the next step's first
+                kf[s % kPf] = kfrag(sk2, s + kPf - kD / 16);
+                vf[s % kPf] = vfrag(st, s + kPf - kD / 16);
+            }
+            // one DMA instruction per four MFMAs: issued together they back up the address unit, and the stalled issue
+            // starves this wave's MFMA pipe
+            if (s & 1) {
+                if (s < 8) dma_k(j + 4, st, s / 2, s / 2 + 1);
+                else dma_v(j + 2, sk2, s / 2 - 4, s / 2 - 3);
+            }
+            sn = mfma_bf16(a, qf[s], sn);
+            O[s & 7] = mfma_bf16(b2, pv[s >> 3], O[s & 7]);
+            if (s < 2) {
+#pragma unroll
+                for (int r = 8 * s; r < 8 * s + 8; ++r) mx = __builtin_fmaxf(mx, sc[r]);
+                __asm__ volatile("" : "+v"(mx));
+            } else if (s == 2) {
+                // the maximum in log2 units (the scale is positive, so it commutes with the maximum and its
+                // rounding); the other half of the wave holds the same queries' other keys.  The reference moves
+                // only when the new maximum exceeds it by more than 8.
+                mx = half_swap_max(mx) * p.scale_log2;
+                grow = mx > m_used + 8.0f;
+                alpha = grow ? __builtin_amdgcn_exp2f(m_used - mx) : 1.0f;
+                if (grow) m_used = mx;
+                __asm__ volatile("" : "+v"(m_used), "+v"(alpha));
+            } else {
+                if (s == 3) lsum *= alpha;
+                if (s <= 5) {
+                    prob(2 * s - 6);
+                    prob(2 * s - 5);
+                } else {
+                    prob(s);
+                }
+                if (s >= 4 && s <= 6) pair(s - 4);              // a step after its exponentials
+                if (s >= 8 && !(s & 1)) pair(s / 2 - 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        pair(7);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            pv[s] = __builtin_bit_cast(bf16x8, u32x4{pw[4 * s], pw[4 * s + 1], pw[4 * s + 2], pw[4 * s + 3]});
+        sc = sn;
+        // O holds tiles up to j - 1; rescaled to the new reference before P of tile j is added
+        if (__builtin_amdgcn_ballot_w64(grow)) {
+#pragma unroll
+            for (int dt = 0; dt < kD / 32; ++dt) O[dt] *= alpha;
+        }
+    }
+    if (first <= last_own) {   // the last tile: O += V P of the tile before, its softmax, O += V P
+        const int t = last_own - first, sv = t % kPSt, svp = (t + 3) % kPSt;
+        fa_wait_vmcnt<0>();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        auto product = [&](int stage) {
+            bf16x8 vf[kPf];
+#pragma unroll
+            for (int i = 0; i < kPf; ++i) vf[i] = vfrag(stage, i);
+#pragma unroll
+            for (int m = 0; m < kD / 16; ++m) {
+                const bf16x8 a = vf[m % kPf];
+                if (m + kPf < kD / 16) vf[m % kPf] = vfrag(stage, m + kPf);
+                __builtin_amdgcn_sched_barrier(0);
+                O[m & 7] = mfma_bf16(a, pv[m >> 3], O[m & 7]);
+            }
+        };
+        product(svp);
+        mask(last_own, sc);
+        float mx = -__builtin_inff();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, sc[r]);
+        mx = half_swap_max(mx) * p.scale_log2;
+        const bool grow = mx > m_used + 8.0f;
+        const float alpha = grow ? __builtin_amdgcn_exp2f(m_used - mx) : 1.0f;
+        if (grow) m_used = mx;
+        lsum *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) prob(r);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pair(i);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            pv[s] = __builtin_bit_cast(bf16x8, u32x4{pw[4 * s], pw[4 * s + 1], pw[4 * s + 2], pw[4 * s + 3]});
+        if (__builtin_amdgcn_ballot_w64(grow)) {
+#pragma unroll
+            for (int dt = 0; dt < kD / 32; ++dt) O[dt] *= alpha;
+        }
+        product(sv);
+    }
     }
     const float ltot = half_swap_sum(lsum);
     if constexpr (SPLIT) {
@@ -649,10 +867,13 @@ int attention_launch(const void *q, long long sbq, long long shq, long long ldq,
         if (rc) return rc;
     }
     if (key_splits == 1) {
-        hipLaunchKernelGGL(fa_fwd_kernel<false>, dim3(HK, B, ntiles_q), dim3(kFaThreads), 0, stream_, p);
+        if ((long long)HK * B * ntiles_q <= kPipeBlocks && Sk >= kPipeKeys)
+            hipLaunchKernelGGL((fa_fwd_kernel<false, true>), dim3(HK, B, ntiles_q), dim3(kFaThreads), 0, stream_, p);
+        else
+            hipLaunchKernelGGL((fa_fwd_kernel<false, false>), dim3(HK, B, ntiles_q), dim3(kFaThreads), 0, stream_, p);
         return mica_err(hipGetLastError());
     }
-    hipLaunchKernelGGL(fa_fwd_kernel<true>, dim3(HK, B, ntiles_q * key_splits), dim3(kFaThreads), 0, stream_, p);
+    hipLaunchKernelGGL((fa_fwd_kernel<true, false>), dim3(HK, B, ntiles_q * key_splits), dim3(kFaThreads), 0, stream_, p);
     rc = mica_err(hipGetLastError());
     if (rc) return rc;
     const long long rows = (long long)B * HQ * Sq;

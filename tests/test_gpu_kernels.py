@@ -1020,6 +1020,31 @@ def test_attention_split_keys_matches_oracle(gpu, B, Sq, Sk, HK, splits):
     assert w_split <= 2.0 * w_one + 1e-3
 
 
+@pytest.mark.parametrize("B,S,P", [
+    (5, 1024, 0),    # 640 workgroups together, 128 alone: the two schedules
+    (17, 250, 640),  # 544 / 32, queries past the last tile's end, the diagonal across two tiles of a prefix's end
+    (16, 263, 1088), # 576 / 36, 9 query blocks, the last 7 rows long
+])
+def test_attention_schedules_agree_bit_for_bit(gpu, B, S, P):
+    """Few workgroups over long keys run the pipelined schedule, more of them the other: the sequences of a batch run
+    together and alone must agree in every bit (the same arithmetic per query)."""
+    from mica_amd.attention import causal_gqa_attention
+
+    note(f"attention schedules B={B} S={S} P={P}")
+    g = torch.Generator(device=gpu).manual_seed(B * S + P)
+    qkv = torch.randn(B, S, 24, 256, generator=g, device=gpu).to(torch.bfloat16)
+    qkv[:, S // 2:] *= 3          # maxima that grow late: the rescale runs beyond the first tiles
+    q, k, v = qkv.split((16, 4, 4), dim=2)
+    pre = None
+    if P:
+        kv = torch.randn(2, P, 4, 256, generator=g, device=gpu).to(torch.bfloat16)
+        pre = (kv[0], kv[1])
+    together = causal_gqa_attention(q, k, v, prefix=pre)
+    for b in range(B):
+        alone = causal_gqa_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], prefix=pre)
+        assert torch.equal(alone[0], together[b]), b
+
+
 @pytest.mark.parametrize("B,P,Sn,Sq,HK,splits,use_len", [
     (3, 64, 96, 96, 1, 1, False),     # continuations of one prefix: every new row a query
     (2, 256, 40, 40, 2, 1, False),    # ragged last tile of the new keys
