@@ -374,6 +374,13 @@ int mica_gdn_chunk(const void *q, long long sbq, int ldq, const void *k, long lo
                    const float *initial_state, float *final_state, void *o, float scale, int B, int T, int HK, int HV,
                    void *workspace, long long workspace_bytes, mica_stream_t stream);
 
+/* mica_gdn_chunk with the gate inside: g and beta of token row m = b T + t and value head h are those of mica_gdn_gate
+ * on a[m lda + h], b[m ldb + h], A_log[h] and dt_bias[h] (same bits as the two calls; nothing is written in between) */
+int mica_gdn_chunk_gate(const void *q, long long sbq, int ldq, const void *k, long long sbk, int ldk, const void *v,
+                        long long sbv, int ldv, const void *a, int lda, const void *b, int ldb, const float *A_log,
+                        const float *dt_bias, const float *initial_state, float *final_state, void *o, float scale,
+                        int B, int T, int HK, int HV, void *workspace, long long workspace_bytes, mica_stream_t stream);
+
 /* bytes of mica_gdn_chunk workspace: B x HV x ceil(T / 64) x 33 KiB (W, U and the in-chunk decays) */
 long long mica_gdn_workspace_bytes(int B, int T, int HV);
 

@@ -67,6 +67,8 @@ SIGNATURES = {
     "mica_causal_conv1d": (_I, [_P, _LL, _I, _P, _P, _I, _I, _P, _P, _P, _LL, _I, _I, _I, _I, _I, _I, _F, _P]),
     "mica_gdn_chunk": (_I, [_P, _LL, _I, _P, _LL, _I, _P, _LL, _I, _P, _P, _I, _P, _P, _P, _F, _I, _I, _I, _I, _P,
                             _LL, _P]),
+    "mica_gdn_chunk_gate": (_I, [_P, _LL, _I, _P, _LL, _I, _P, _LL, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _F, _I, _I, _I,
+                                 _I, _P, _LL, _P]),
     "mica_gdn_workspace_bytes": (_LL, [_I, _I, _I]),
     "mica_gated_rmsnorm_quant": (_I, [_P, _I, _P, _I, _P, _F, _P, _I, _P, _I, _P, _I, _I, _P]),
     "mica_gdn_gate": (_I, [_P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _P]),
@@ -75,8 +77,8 @@ SIGNATURES = {
 # functions of libmica_amd.so that the native launch path calls
 NATIVE_FNS = ("mica_act_quant", "mica_mm_i8", "mica_rmsnorm_quant", "mica_rmsnorm_quant_multi",
               "mica_attention_prefix_workspace_bytes", "mica_attention_fwd", "mica_attention_fwd_prefix",
-              "mica_causal_conv1d", "mica_gdn_chunk", "mica_gdn_workspace_bytes", "mica_gdn_gate",
-              "mica_gated_rmsnorm_quant")
+              "mica_causal_conv1d", "mica_gdn_chunk", "mica_gdn_chunk_gate", "mica_gdn_workspace_bytes",
+              "mica_gdn_gate", "mica_gated_rmsnorm_quant")
 
 
 class _NotLoaded:

@@ -45,6 +45,7 @@ struct Abi {
     MICA_FN(attention_fwd_prefix)
     MICA_FN(causal_conv1d)
     MICA_FN(gdn_chunk)
+    MICA_FN(gdn_chunk_gate)
     MICA_FN(gdn_workspace_bytes)
     MICA_FN(gdn_gate)
     MICA_FN(gated_rmsnorm_quant)
@@ -394,51 +395,72 @@ bool heads(const Call &c, const Tensor &t, int64_t B, int64_t T, int64_t H) {
            t.scalar_type() == at::kBFloat16 && t.stride(3) == 1 && t.stride(2) == 128 && on(c, t) && aligned(t);
 }
 
-// gdn_chunk(q, k, v, g, beta, scale, initial state, want final state) -> (o, final state or None)
-PyObject *py_gdn_chunk(PyObject *, PyObject *const *a, Py_ssize_t nargs) {
-    HANDLE_TH_ERRORS
-    MICA_ARGS(8)
-    const Tensor *q, *k, *v, *g, *beta, *h0;
-    Call c;
-    if (!plain(a[0], &q) || !plain(a[1], &k) || !plain(a[2], &v) || !plain(a[3], &g) || !plain(a[4], &beta) ||
-        !plain_opt(a[6], &h0) || !enter(*q, c))
-        return none();
-    const double scale = PyFloat_AsDouble(a[5]);
-    if (PyErr_Occurred()) return nullptr;
-    if (q->dim() != 4 || v->dim() != 4) return none();
-    const int64_t B = q->size(0), T = q->size(1), HK = q->size(2), HV = v->size(2);
-    if (HK < 1 || HV % HK || !heads(c, *q, B, T, HK) || !heads(c, *k, B, T, HK) || !heads(c, *v, B, T, HV)) return none();
-    if (!vec_f32(c, *g, B * T * HV) || g->dim() != 3 || g->size(0) != B || g->size(1) != T) return none();
-    const int bd = code(beta->scalar_type());
-    if ((bd != MICA_BF16 && bd != MICA_FP32) || beta->sizes() != g->sizes() || !beta->is_contiguous() || !on(c, *beta))
-        return none();
-    if (h0 && (!vec_f32(c, *h0, B * HV * 128 * 128) || h0->dim() != 4 || h0->size(0) != B || h0->size(1) != HV ||
-               h0->size(2) != 128 || !aligned(*h0)))
-        return none();
-    const long long nbytes = abi.gdn_workspace_bytes((int)B, (int)T, (int)HV);
-    if (nbytes < 0) return none();
-    const bool want = PyObject_IsTrue(a[7]);
-    Tensor hT;
-    if (want) hT = make(c, {B, HV, 128, 128}, at::kFloat);
-    const Tensor o = make(c, {B, T, HV, 128}, at::kBFloat16), ws = make(c, {std::max<int64_t>(nbytes, 16)}, at::kByte);
-    auto sb = [&](const Tensor &t) { return (long long)(B > 1 ? t.stride(0) : T * t.stride(1)); };
-    const int rc = launch([&] {
-        return abi.gdn_chunk(q->data_ptr(), sb(*q), (int)q->stride(1), k->data_ptr(), sb(*k), (int)k->stride(1), v->data_ptr(),
-                             sb(*v), (int)v->stride(1), (const float *)g->data_ptr(), beta->data_ptr(), bd,
-                             (const float *)ptr(h0), want ? (float *)hT.data_ptr() : nullptr, o.data_ptr(), (float)scale,
-                             (int)B, (int)T, (int)HK, (int)HV, ws.data_ptr(), nbytes, c.stream);
-    });
-    if (rc) return bad(rc);
-    return pack({wrap(o), want ? wrap(hT) : new_none()});
-    END_HANDLE_TH_ERRORS
-}
-
 // rows [M, N] of t over its last axis, when they are evenly spaced
 bool rows_of(const Tensor &t, int64_t &M, int64_t &N, int64_t &ld) {
     if (t.dim() != 2 || t.stride(1) != 1) return false;
     M = t.size(0), N = t.size(1), ld = t.stride(0);
     return true;
 }
+
+// gdn_chunk(q, k, v, g, beta, scale, initial state, want final state), or with (a, b, A_log, dt_bias) in the place of
+// (g, beta) -> (o, final state or None)
+PyObject *chunk(PyObject *const *a, Py_ssize_t nargs, bool gate) {
+    HANDLE_TH_ERRORS
+    MICA_ARGS(gate ? 10 : 8)
+    PyObject *const *rest = a + (gate ? 7 : 5);
+    const Tensor *q, *k, *v, *g, *beta, *A = nullptr, *dt = nullptr, *h0;
+    Call c;
+    if (!plain(a[0], &q) || !plain(a[1], &k) || !plain(a[2], &v) || !plain(a[3], &g) || !plain(a[4], &beta) ||
+        (gate && (!plain(a[5], &A) || !plain(a[6], &dt))) || !plain_opt(rest[1], &h0) || !enter(*q, c))
+        return none();
+    const double scale = PyFloat_AsDouble(rest[0]);
+    if (PyErr_Occurred()) return nullptr;
+    if (q->dim() != 4 || v->dim() != 4) return none();
+    const int64_t B = q->size(0), T = q->size(1), HK = q->size(2), HV = v->size(2);
+    if (HK < 1 || HV % HK || !heads(c, *q, B, T, HK) || !heads(c, *k, B, T, HK) || !heads(c, *v, B, T, HV)) return none();
+    int bd = 0;
+    int64_t lda = 0, ldb = 0;
+    if (gate) { // g and beta are the rows a and b
+        int64_t M, N, M2, N2;
+        if (!rows_of(*g, M, N, lda) || !rows_of(*beta, M2, N2, ldb) || M != B * T || M2 != M || N != HV || N2 != HV ||
+            g->scalar_type() != at::kBFloat16 || beta->scalar_type() != at::kBFloat16 || !on(c, *g) || !on(c, *beta) ||
+            !vec_f32(c, *A, HV) || !vec_f32(c, *dt, HV))
+            return none();
+    } else {
+        if (!vec_f32(c, *g, B * T * HV) || g->dim() != 3 || g->size(0) != B || g->size(1) != T) return none();
+        bd = code(beta->scalar_type());
+        if ((bd != MICA_BF16 && bd != MICA_FP32) || beta->sizes() != g->sizes() || !beta->is_contiguous() || !on(c, *beta))
+            return none();
+    }
+    if (h0 && (!vec_f32(c, *h0, B * HV * 128 * 128) || h0->dim() != 4 || h0->size(0) != B || h0->size(1) != HV ||
+               h0->size(2) != 128 || !aligned(*h0)))
+        return none();
+    const long long nbytes = abi.gdn_workspace_bytes((int)B, (int)T, (int)HV);
+    if (nbytes < 0) return none();
+    const bool want = PyObject_IsTrue(rest[2]);
+    Tensor hT;
+    if (want) hT = make(c, {B, HV, 128, 128}, at::kFloat);
+    const Tensor o = make(c, {B, T, HV, 128}, at::kBFloat16), ws = make(c, {std::max<int64_t>(nbytes, 16)}, at::kByte);
+    auto sb = [&](const Tensor &t) { return (long long)(B > 1 ? t.stride(0) : T * t.stride(1)); };
+    float *hp = want ? (float *)hT.data_ptr() : nullptr;
+    const int rc = launch([&] {
+        if (gate)
+            return abi.gdn_chunk_gate(q->data_ptr(), sb(*q), (int)q->stride(1), k->data_ptr(), sb(*k), (int)k->stride(1),
+                                      v->data_ptr(), sb(*v), (int)v->stride(1), g->data_ptr(), (int)lda, beta->data_ptr(),
+                                      (int)ldb, (const float *)A->data_ptr(), (const float *)dt->data_ptr(),
+                                      (const float *)ptr(h0), hp, o.data_ptr(), (float)scale, (int)B, (int)T, (int)HK,
+                                      (int)HV, ws.data_ptr(), nbytes, c.stream);
+        return abi.gdn_chunk(q->data_ptr(), sb(*q), (int)q->stride(1), k->data_ptr(), sb(*k), (int)k->stride(1), v->data_ptr(),
+                             sb(*v), (int)v->stride(1), (const float *)g->data_ptr(), beta->data_ptr(), bd,
+                             (const float *)ptr(h0), hp, o.data_ptr(), (float)scale, (int)B, (int)T, (int)HK, (int)HV,
+                             ws.data_ptr(), nbytes, c.stream);
+    });
+    if (rc) return bad(rc);
+    return pack({wrap(o), want ? wrap(hT) : new_none()});
+    END_HANDLE_TH_ERRORS
+}
+PyObject *py_gdn_chunk(PyObject *, PyObject *const *a, Py_ssize_t n) { return chunk(a, n, false); }
+PyObject *py_gdn_chunk_gate(PyObject *, PyObject *const *a, Py_ssize_t n) { return chunk(a, n, true); }
 
 // gdn_gate(a, b, A_log, dt_bias) -> (g, beta), a and b [M, HV]
 PyObject *py_gdn_gate(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
@@ -507,6 +529,7 @@ PyObject *py_bind(PyObject *, PyObject *d) {
     MICA_FN(attention_fwd_prefix)
     MICA_FN(causal_conv1d)
     MICA_FN(gdn_chunk)
+    MICA_FN(gdn_chunk_gate)
     MICA_FN(gdn_workspace_bytes)
     MICA_FN(gdn_gate)
     MICA_FN(gated_rmsnorm_quant)
@@ -552,6 +575,7 @@ PyMethodDef kMethods[] = {
     MICA_DEF("attention", py_attention),
     MICA_DEF("conv", py_conv),
     MICA_DEF("gdn_chunk", py_gdn_chunk),
+    MICA_DEF("gdn_chunk_gate", py_gdn_chunk_gate),
     MICA_DEF("gdn_gate", py_gdn_gate),
     MICA_DEF("gated_norm", py_gated_norm),
     {"bind", py_bind, METH_O, nullptr},

@@ -178,6 +178,9 @@ struct GdnParams {
     const uint16_t *v; long long sbv; int ldv;  // bf16 [B][T][HV][128]
     const float *g;                             // fp32 [B][T][HV]
     const void *beta; int beta_dtype;           // [B][T][HV], bf16 or fp32
+    // instead of g and beta (then null): the gate's inputs, bf16 rows [B T][HV], fp32 [HV]
+    const uint16_t *ga, *gb; int ldga, ldgb;
+    const float *A_log, *dt_bias;
     const float *h0;                            // fp32 [B][HV][128][128] or null
     float *hT;                                  // fp32 [B][HV][128][128] or null
     uint16_t *o;                                // bf16 [B][T][HV][128]
@@ -186,6 +189,17 @@ struct GdnParams {
     float scale;
     int B, T, HK, HV, NT;
 };
+
+// The GDN layer's decay and write strength per token and value head (fork.py:124-125):
+//   g = -exp(A_log[h]) * softplus(f32(a) + dt_bias[h])   (softplus(x) = x above 20, else log1p(exp(x)),
+//                                                         torch's threshold), fp32
+//   beta = bf16(sigmoid(f32(b)))                         (torch's bf16 sigmoid: fp32 math, one rounding)
+MICA_DEVICE float gate_decay(uint16_t a, float A_log, float dt_bias) {
+    const float x = bf16_to_f32(a) + dt_bias;
+    const float sp = x > 20.0f ? x : log1pf(expf(x));
+    return -expf(A_log) * sp;
+}
+MICA_DEVICE uint16_t gate_strength(uint16_t b) { return f32_to_bf16(1.0f / (1.0f + expf(-bf16_to_f32(b)))); }
 
 // per (b, h, chunk) workspace blocks
 MICA_DEVICE long chunk_id(const GdnParams &p, int b, int h, int c) { return ((long)b * p.HV + h) * p.NT + c; }
@@ -278,8 +292,14 @@ __global__ __launch_bounds__(kGdnThreads) void gdn_prep_kernel(GdnParams p) {
         float bv = 0.0f;
         if (t < p.T) {
             const long gi = ((long)b * p.T + t) * p.HV + h;
-            gval = p.g[gi];
-            bv = load_as_f32(p.beta, p.beta_dtype, gi);
+            if (p.ga != nullptr) {
+                const long m = (long)b * p.T + t;
+                gval = gate_decay(p.ga[m * p.ldga + h], p.A_log[h], p.dt_bias[h]);
+                bv = bf16_to_f32(gate_strength(p.gb[m * p.ldgb + h]));
+            } else {
+                gval = p.g[gi];
+                bv = load_as_f32(p.beta, p.beta_dtype, gi);
+            }
         }
         Gs[tid] = gval;
         Bs[tid] = bv;
@@ -832,21 +852,15 @@ __global__ __launch_bounds__(64 * kGnWaves) void gated_norm_quant_kernel(GatedNo
     if (lane == 0) p.s[row] = s;
 }
 
-// The GDN layer's decay and write strength per token and value head (fork.py:124-125):
-//   g = -exp(A_log[h]) * softplus(f32(a) + dt_bias[h])   (softplus(x) = x above 20, else log1p(exp(x)),
-//                                                         torch's threshold), fp32
-//   beta = bf16(sigmoid(f32(b)))                         (torch's bf16 sigmoid: fp32 math, one rounding)
-// One thread per (token, head); a and b are the bf16 outputs of in_proj_a / in_proj_b.
+// gate_decay and gate_strength, one thread per (token, head); a and b are the bf16 outputs of in_proj_a / in_proj_b.
 __global__ __launch_bounds__(256) void gate_kernel(const uint16_t *a, int lda, const uint16_t *b, int ldb,
                                                    const float *A_log, const float *dt_bias, float *g,
                                                    uint16_t *beta, int M, int HV) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i >= (long)M * HV) return;
     const int m = (int)(i / HV), h = (int)(i - (long)m * HV);
-    const float x = bf16_to_f32(a[(long)m * lda + h]) + dt_bias[h];
-    const float sp = x > 20.0f ? x : log1pf(expf(x));
-    g[i] = -expf(A_log[h]) * sp;
-    beta[i] = f32_to_bf16(1.0f / (1.0f + expf(-bf16_to_f32(b[(long)m * ldb + h]))));
+    g[i] = gate_decay(a[(long)m * lda + h], A_log[h], dt_bias[h]);
+    beta[i] = gate_strength(b[(long)m * ldb + h]);
 }
 
 // dst = src (or zeros when src is null): the final state of an empty scan
@@ -914,15 +928,18 @@ extern "C" long long mica_gdn_workspace_bytes(int B, int T, int HV) {
     return gdn_ws_bytes(B, T, HV);
 }
 
-extern "C" int mica_gdn_chunk(const void *q, long long sbq, int ldq, const void *k, long long sbk, int ldk,
-                              const void *v, long long sbv, int ldv, const float *g, const void *beta,
-                              int beta_dtype, const float *initial_state, float *final_state, void *o, float scale,
-                              int B, int T, int HK, int HV, void *workspace, long long workspace_bytes,
-                              mica_stream_t stream) {
-    if (beta_dtype != MICA_BF16 && beta_dtype != MICA_FP32) return MICA_MISS_DTYPE;
+namespace {
+
+// p.g, p.beta, p.beta_dtype or the gate's inputs come set; the other arguments as in mica_gdn_chunk
+int gdn_chunk_launch(GdnParams p, const void *q, long long sbq, int ldq, const void *k, long long sbk, int ldk,
+                     const void *v, long long sbv, int ldv, const float *initial_state, float *final_state, void *o,
+                     float scale, int B, int T, int HK, int HV, void *workspace, long long workspace_bytes,
+                     mica_stream_t stream) {
     if (B < 0 || T < 0 || HK <= 0 || HV <= 0 || HV % HK != 0) return MICA_MISS_SHAPE;
     // empty inputs have no token data (their pointers may be NULL)
-    if (B > 0 && T > 0 && (q == nullptr || k == nullptr || v == nullptr || g == nullptr || beta == nullptr || o == nullptr))
+    const bool gated = p.ga != nullptr && p.gb != nullptr && p.A_log != nullptr && p.dt_bias != nullptr;
+    if (B > 0 && T > 0 && (q == nullptr || k == nullptr || v == nullptr || o == nullptr ||
+                           (!gated && (p.g == nullptr || p.beta == nullptr))))
         return MICA_MISS_ARG;
     if (ldq < HK * kDk || ldk < HK * kDk || ldv < HV * kDv || ldq % 8 || ldk % 8 || ldv % 8 || sbq % 8 || sbk % 8 ||
         sbv % 8 || sbq < (long long)T * ldq || sbk < (long long)T * ldk || sbv < (long long)T * ldv)
@@ -945,11 +962,9 @@ extern "C" int mica_gdn_chunk(const void *q, long long sbq, int ldq, const void 
         return 0;
     }
     if (workspace == nullptr || workspace_bytes < gdn_ws_bytes(B, T, HV)) return MICA_MISS_ARG;
-    GdnParams p{};
     p.q = (const uint16_t *)q; p.sbq = sbq; p.ldq = ldq;
     p.k = (const uint16_t *)k; p.sbk = sbk; p.ldk = ldk;
     p.v = (const uint16_t *)v; p.sbv = sbv; p.ldv = ldv;
-    p.g = g; p.beta = beta; p.beta_dtype = beta_dtype;
     p.h0 = initial_state; p.hT = final_state; p.o = (uint16_t *)o; p.scale = scale;
     p.B = B; p.T = T; p.HK = HK; p.HV = HV; p.NT = (T + kC - 1) / kC;
     const long long blocks = (long long)B * HV * p.NT;
@@ -970,6 +985,36 @@ extern "C" int mica_gdn_chunk(const void *q, long long sbq, int ldq, const void 
     else if (pairs * 2 <= cus) hipLaunchKernelGGL((gdn_scan_kernel<1, 8>), dim3(HV, B, 2), dim3(512), 0, st, p);
     else hipLaunchKernelGGL((gdn_scan_kernel<2, 8>), dim3(HV, B, 1), dim3(512), 0, st, p);
     return mica_err(hipGetLastError());
+}
+
+}  // namespace
+
+extern "C" int mica_gdn_chunk(const void *q, long long sbq, int ldq, const void *k, long long sbk, int ldk,
+                              const void *v, long long sbv, int ldv, const float *g, const void *beta,
+                              int beta_dtype, const float *initial_state, float *final_state, void *o, float scale,
+                              int B, int T, int HK, int HV, void *workspace, long long workspace_bytes,
+                              mica_stream_t stream) {
+    if (beta_dtype != MICA_BF16 && beta_dtype != MICA_FP32) return MICA_MISS_DTYPE;
+    GdnParams p{};
+    p.g = g; p.beta = beta; p.beta_dtype = beta_dtype;
+    return gdn_chunk_launch(p, q, sbq, ldq, k, sbk, ldk, v, sbv, ldv, initial_state, final_state, o, scale, B, T, HK, HV,
+                            workspace, workspace_bytes, stream);
+}
+
+extern "C" int mica_gdn_chunk_gate(const void *q, long long sbq, int ldq, const void *k, long long sbk, int ldk,
+                                   const void *v, long long sbv, int ldv, const void *a, int lda, const void *b,
+                                   int ldb, const float *A_log, const float *dt_bias, const float *initial_state,
+                                   float *final_state, void *o, float scale, int B, int T, int HK, int HV,
+                                   void *workspace, long long workspace_bytes, mica_stream_t stream) {
+    if (B > 0 && T > 0 && (a == nullptr || b == nullptr || A_log == nullptr || dt_bias == nullptr)) return MICA_MISS_ARG;
+    if (lda < HV || ldb < HV) return MICA_MISS_STRIDE;
+    if ((long long)B * T * lda >= (1LL << 31) || (long long)B * T * ldb >= (1LL << 31)) return MICA_MISS_RANGE;
+    GdnParams p{};
+    p.ga = (const uint16_t *)a; p.ldga = lda;
+    p.gb = (const uint16_t *)b; p.ldgb = ldb;
+    p.A_log = A_log; p.dt_bias = dt_bias;
+    return gdn_chunk_launch(p, q, sbq, ldq, k, sbk, ldk, v, sbv, ldv, initial_state, final_state, o, scale, B, T, HK, HV,
+                            workspace, workspace_bytes, stream);
 }
 
 extern "C" int mica_gated_rmsnorm_quant(const void *x, int ldx, const void *z, int ldz, const void *w, float eps,

@@ -26,6 +26,10 @@ from .int8_kernels import _aligned, _gpu_ok, _launched, _native, _on, _stream
 
 HEAD_DIM = 128
 CHUNK = 64
+# (chunk, value head) pairs up to which the gate is formed inside the scan's preparation.  Measured on MI355X, 32 heads
+# (us, two calls / one): 1 x 64 16.5 / 14.6, 1 x 333 33.6 / 31.3, 8 x 300 52.6 / 49.9, 4 x 1024 (2048 pairs) 82.3 / 81.1,
+# 8 x 1024 (4096) 146.6 / 143.7, 8 x 1500 (6144) 205.4 / 206.0, 8 x 2048 (8192) 274.5 / 279.8
+GATE_CHUNKS = 4096
 
 
 def _need_gpu(*ts):
@@ -215,6 +219,23 @@ def gdn_gate(a, b, A_log, dt_bias):
     return g.view(a.shape), beta.view(a.shape)
 
 
+def chunk_gated_delta_rule_gate(q, k, v, a, b, A_log, dt_bias, scale=None, initial_state=None,
+                                output_final_state=False):
+    """gdn_gate and chunk_gated_delta_rule in one step: a, b are bf16 rows [B * T, HV], the decays and write strengths
+    are formed where the scan's preparation reads them (same bits as the two calls, one launch and 6 bytes per token
+    and head of traffic less), for up to GATE_CHUNKS (chunk, head) pairs; past that the two calls, whose reads of a and
+    b are coalesced.  Returns (o, final_state or None)."""
+    B, T = q.shape[:2]
+    if B * (-(-T // CHUNK)) * v.shape[2] <= GATE_CHUNKS:
+        r = _lib.FAST.gdn_chunk_gate(q, k, v, a, b, A_log, dt_bias, HEAD_DIM ** -0.5 if scale is None else float(scale),
+                                     initial_state, output_final_state)
+        if r is not None:
+            return _native(r, "mica_gdn_chunk_gate")
+    g, beta = gdn_gate(a, b, A_log, dt_bias)
+    return chunk_gated_delta_rule(q, k, v, g.view(B, T, -1), beta.view(B, T, -1), scale, initial_state,
+                                  output_final_state)
+
+
 def gated_rmsnorm_quant(x, z, weight, eps: float = 1e-6, want_y: bool = False):
     """attn.norm(x, z) over 128-wide heads, then per-token INT8 (half-even) of the [.., HV * 128] row.
     Returns (q int8 [M, N], s fp32 [M]) or, with want_y, (q, s, y bf16 [M, N])."""
@@ -251,7 +272,8 @@ class GDNLayer(torch.nn.Module):
       1. input RMSNorm, quantized per token once for the four projections (in_proj_qkv, in_proj_z,
          in_proj_b, in_proj_a; each a QLinear with its own SmoothQuant factors)  -> 1 + 4 launches
       2. causal conv + SiLU over the q / k / v channels, q / k l2-normalised  -> 1 launch
-      3. g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b)  (fork.py:124-125)  -> 1 launch
+      3. g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b)  (fork.py:124-125), formed by the next
+         step (a launch of its own for a trace)
       4. chunked gated delta rule  -> 2 launches
       5. gated RMSNorm fused with out_proj's quantisation, out_proj GEMM with the residual add in its
          epilogue  -> 2 launches
@@ -285,10 +307,14 @@ class GDNLayer(torch.nn.Module):
         conv, conv_state = conv if keep else (conv, None)
         x = conv.transpose(1, 2)                            # [B, T, C] (contiguous memory)
         q, k, v = x.view(batch, T, -1, HEAD_DIM).split((self.hk, self.hk, self.hv), dim=2)
-        g, beta = gdn_gate(a, b, self.A_log, self.dt_bias)
-        o, rec = chunk_gated_delta_rule(q, k, v, g.view(batch, T, self.hv), beta.view(batch, T, self.hv),
-                                        initial_state=None if initial is None else initial[1],
-                                        output_final_state=keep)
+        rec0 = None if initial is None else initial[1]
+        if trace is None:
+            o, rec = chunk_gated_delta_rule_gate(q, k, v, a, b, self.A_log, self.dt_bias, initial_state=rec0,
+                                                 output_final_state=keep)
+        else:
+            g, beta = gdn_gate(a, b, self.A_log, self.dt_bias)
+            o, rec = chunk_gated_delta_rule(q, k, v, g.view(batch, T, self.hv), beta.view(batch, T, self.hv),
+                                            initial_state=rec0, output_final_state=keep)
         qo, so = gated_rmsnorm_quant(o.view(batch * T, -1), z, self.norm_z_weight, self.z_eps)
         out = self.out_proj.forward_quantized(qo, so, residual=h)
         if trace is not None:

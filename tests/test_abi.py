@@ -229,6 +229,27 @@ def test_gdn_chunk_rejects():
     assert lib.mica_gdn_workspace_bytes(8, 2048, 32) == 8 * 32 * 32 * (2 * 64 * 128 * 2 + 64 * 4)
 
 
+def test_gdn_chunk_gate_rejects():
+    lib = _lib.load()
+    D = 128
+    # (q, sbq, ldq, k, sbk, ldk, v, sbv, ldv, a, lda, b, ldb, A_log, dt_bias, h0, hT, o, scale, B, T, HK, HV, ws, bytes)
+    ok = [A16, 8 * 2 * D, 2 * D, A16, 8 * 2 * D, 2 * D, A16, 8 * 4 * D, 4 * D, A16, 4, A16, 4, A16, A16, None, None, A16,
+          0.1, 1, 8, 2, 4, A16, 1 << 30]
+
+    def with_(**kw):
+        a = list(ok)
+        for i, v in kw.items():
+            a[int(i[1:])] = v
+        return lib.mica_gdn_chunk_gate(*a, None)
+
+    assert with_(a9=None) == 6            # NULL gate input
+    assert with_(a13=None) == 6           # NULL A_log
+    assert with_(a10=3) == 4              # gate rows shorter than the heads
+    assert with_(a22=3) == 1              # HV not a multiple of HK
+    assert with_(a23=None) == 6           # no workspace
+    assert with_(a19=0) == 0              # no sequences
+
+
 def test_gated_rmsnorm_quant_rejects():
     lib = _lib.load()
     # (x, ldx, z, ldz, w, eps, y, ldy, q, ldq, s, M, N)

@@ -227,3 +227,22 @@ def test_gdn_gate_matches_oracle(gpu, M, HV):
     wide = torch.cat([a, b], 1).to(gpu)
     g2, b2 = gdn.gdn_gate(wide[:, :HV], wide[:, HV:], A_log.to(gpu), dt.to(gpu))
     assert torch.equal(g2, gg) and torch.equal(b2, beta)
+
+
+@pytest.mark.parametrize("B,T,HK,HV", [(1, 1, 1, 1), (2, 64, 2, 4), (3, 70, 2, 4), (1, 333, 16, 32)])
+def test_gdn_gate_inside_the_scan_equals_the_two_calls(gpu, B, T, HK, HV):
+    """chunk_gated_delta_rule_gate forms the decays and write strengths where the preparation reads them: the bits of
+    gdn_gate followed by chunk_gated_delta_rule, on strided rows, from and to a state."""
+    from mica_amd import gdn
+
+    g = torch.Generator(device=gpu).manual_seed(B * 1000 + T)
+    rn = lambda *sh: torch.randn(*sh, generator=g, device=gpu).to(torch.bfloat16)  # noqa: E731
+    q, k, v = rn(B, T, HK, 128) * 0.09, rn(B, T, HK, 128) * 0.09, rn(B, T, HV, 128)
+    ab = rn(B * T, 2 * HV + 8) * 4
+    a, b = ab[:, :HV], ab[:, HV:2 * HV]
+    A, dt = torch.rand(HV, generator=g, device=gpu) * 2 - 1, torch.randn(HV, generator=g, device=gpu)
+    h0 = torch.randn(B, HV, 128, 128, generator=g, device=gpu)
+    gg, beta = gdn.gdn_gate(a, b, A, dt)
+    want = gdn.chunk_gated_delta_rule(q, k, v, gg.view(B, T, HV), beta.view(B, T, HV), None, h0, True)
+    got = gdn.chunk_gated_delta_rule_gate(q, k, v, a, b, A, dt, None, h0, True)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
