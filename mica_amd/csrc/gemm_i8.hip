@@ -779,7 +779,7 @@ int mm_i8_run(const int8_t *A, int lda, const int8_t *B, int ldb, const float *s
         int rc = 0;
         if (thin_launch(p, epilogue, out_dtype, cus, bias != nullptr, residual != nullptr, st, &rc)) return rc;
     }
-    // Few tiles and a long K (a short request's down projection, e.g. 128 x 2560 x 9728: 16 tiles of
+    // Few tiles and a long K that no small tile covers in one round (e.g. 512 x 2560 x 9728: 64 tiles of
     // 128 x 160 on 256 CUs): with a workspace, one round of 128-row tiles split along K into `parts`
     // pieces whose int32 partial sums each tile's last part adds (agpr_split_launch; same bits as every
     // other schedule).  The hand-off costs ~5 us (the partial sums' write-through, the arrival count,

@@ -14,7 +14,7 @@
 //   2560 x 4096 + residual   13.0 ->  4.4   13.3 ->  5.7   14.2 ->  7.4   14.4 ->  9.3
 //   6144 x 2560              19.5 ->  5.9   19.8 ->  8.6   23.6 -> 10.3   21.6 -> 13.2
 //   12352 x 2560             20.1 ->  8.6   20.7 -> 11.8   24.5 -> 15.3   23.3 -> 19.2
-//   19456 x 2560 SiLU        15.3 -> 14.0   17.8 -> 16.1   19.9 -> 19.4   (29.7, no one-round tile: not taken)
+//   19456 x 2560 SiLU        15.3 -> 14.0   17.8 -> 16.1   19.9 -> 19.4   (29.7 -> 29.8 at 224: not taken)
 // Tried without gain: fragments loaded straight to registers (16 rows x 64 bytes per load: 64 clocks each in
 // the address unit, 16 bytes per clock), a wave that touches the weights ahead of the DMA (they are already as
 // deep in flight as the feed takes them), and a different K start per tile.
@@ -97,6 +97,33 @@ MICA_DEVICE void read_frags<2, 4>(v4i (&x)[2][2], v4i (&w)[2][4], uint32_t x0, u
                  : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(w[0][2]),
                    "=&v"(w[0][3]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(w[1][0]), "=&v"(w[1][1]),
                    "=&v"(w[1][2]), "=&v"(w[1][3])
+                 : [x0] "v"(x0), [x1] "v"(x1), [w0] "v"(w0), [w1] "v"(w1));
+}
+template <>
+MICA_DEVICE void read_frags<5, 2>(v4i (&x)[2][5], v4i (&w)[2][2], uint32_t x0, uint32_t x1, uint32_t w0,
+                                  uint32_t w1) {
+    asm volatile(MICA_RD(0, x0, 0) MICA_RD(1, x0, 1) MICA_RD(2, x0, 2) MICA_RD(3, x0, 3)
+                 MICA_RD(4, x0, 4) MICA_RD(5, w0, 0) MICA_RD(6, w0, 1)
+                 MICA_RD(7, x1, 0) MICA_RD(8, x1, 1) MICA_RD(9, x1, 2) MICA_RD(10, x1, 3)
+                 MICA_RD(11, x1, 4) MICA_RD(12, w1, 0) MICA_RD(13, w1, 1)
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[0][2]), "=&v"(x[0][3]), "=&v"(x[0][4]),
+                   "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(x[1][2]),
+                   "=&v"(x[1][3]), "=&v"(x[1][4]), "=&v"(w[1][0]), "=&v"(w[1][1])
+                 : [x0] "v"(x0), [x1] "v"(x1), [w0] "v"(w0), [w1] "v"(w1));
+}
+template <>
+MICA_DEVICE void read_frags<6, 2>(v4i (&x)[2][6], v4i (&w)[2][2], uint32_t x0, uint32_t x1, uint32_t w0,
+                                  uint32_t w1) {
+    asm volatile(MICA_RD(0, x0, 0) MICA_RD(1, x0, 1) MICA_RD(2, x0, 2) MICA_RD(3, x0, 3)
+                 MICA_RD(4, x0, 4) MICA_RD(5, x0, 5) MICA_RD(6, w0, 0) MICA_RD(7, w0, 1)
+                 MICA_RD(8, x1, 0) MICA_RD(9, x1, 1) MICA_RD(10, x1, 2) MICA_RD(11, x1, 3)
+                 MICA_RD(12, x1, 4) MICA_RD(13, x1, 5) MICA_RD(14, w1, 0) MICA_RD(15, w1, 1)
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[0][2]), "=&v"(x[0][3]), "=&v"(x[0][4]),
+                   "=&v"(x[0][5]), "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]),
+                   "=&v"(x[1][2]), "=&v"(x[1][3]), "=&v"(x[1][4]), "=&v"(x[1][5]), "=&v"(w[1][0]),
+                   "=&v"(w[1][1])
                  : [x0] "v"(x0), [x1] "v"(x1), [w0] "v"(w0), [w1] "v"(w1));
 }
 #undef MICA_RD
@@ -289,33 +316,48 @@ constexpr ThinTile thin_entry() {
     else
         return ThinTile{C::BM, C::BN, C::WK, thin_launch_out<C, MICA_EPI_SCALE>, nullptr};
 }
+// (SiLU only: half the columns of a tile are outputs there, so a round holds wider tiles; for the plain epilogue
+// 131 x 12352 x 2560 took 19.4 us on 80 x 160 tiles against 15.6 on 128 x 128)
+template <class C>
+constexpr ThinTile thin_silu() {
+    return ThinTile{C::BM, C::BN, C::WK, nullptr, thin_launch_out<C, MICA_EPI_SILU_MUL>};
+}
 const ThinTile kThinTiles[] = {
     thin_entry<TCfg<16, 16, 4, 1, 1, 8>, false>(), thin_entry<TCfg<16, 32, 4, 1, 1, 6>>(),
     thin_entry<TCfg<16, 64, 4, 1, 2, 3>>(),        thin_entry<TCfg<32, 32, 4, 2, 1, 4>>(),
     thin_entry<TCfg<64, 32, 4, 2, 1, 3>>(),        thin_entry<TCfg<32, 64, 4, 1, 2, 3>>(),
     thin_entry<TCfg<64, 64, 2, 2, 2, 4>>(),        thin_entry<TCfg<32, 128, 2, 2, 2, 3>>(),
     thin_entry<TCfg<128, 64, 1, 4, 2, 5>>(),       thin_entry<TCfg<64, 128, 1, 2, 4, 5>>(),
-    thin_entry<TCfg<128, 128, 1, 4, 2, 4>>(),
+    thin_entry<TCfg<128, 128, 1, 4, 2, 4>>(),      thin_silu<TCfg<80, 160, 1, 1, 5, 5>>(),
+    thin_silu<TCfg<96, 192, 1, 1, 6, 4>>(),
 };
 
-// The tile that streams the fewest bytes per CU among those that cover the output in one round and whose waves'
-// K shares divide K; none past 384 rows or 1.25 MB per tile.  Measured against the other kernels (us, cold weights,
-// other / this): 384 x 6144 x 2560 21.3 / 17.4, 384 x 10240 x 2560 19.1 / 18.8, 256 x 2560 x 9728 27.4 / 24.4; past
-// the lines 512 x 6144 x 2560 16.5 / 18.7 (rows), 512 x 2560 x 9728 28.9 / 35 (bytes, 128 x 64 tiles), 384 x 12352 x
-// 2560 19.6 / 33.9 and SiLU 200 x 19456 x 2560 27.7 / 30.6 (more than one round).
+// The tile that streams the fewest bytes per CU among those that cover the output in one round (128 x 128 with SiLU:
+// or in two, the second three quarters full) and whose waves' K shares divide K; none past 384 rows or 1.25 MB a
+// round; with SiLU, tiles of 128 x 128 and more want K >= 2048 (2560 past two rows of tiles) and the two of SiLU's own
+// at most two rows of tiles.  Measured against the other kernels (us, cold weights, other / this): 384 x 6144 x 2560
+// 21.5 / 17.8, 384 x 2560 x 9728 46.6 / 24.0, 8192 x 1024 at 40 rows 9.7 / 5.3, at 384 10.8 / 10.1, SiLU x 19456 x 2560
+// at 131 rows 26.3 / 20.2, 192 28.7 / 23.4, 300 38.1 / 30.7 (two rounds); past the lines 512 x 6144 x 2560 16.5 / 18.7
+// (rows), 512 x 2560 x 9728 28.9 / 35 (bytes, 128 x 64 tiles), 384 x 12352 x 2560 19.6 / 33.9 (1.1 rounds), SiLU 224 x
+// 24576 x 4096 42.7 / 47.8 (1.5), 131 x 12288 x 1024 9.0 / 10.3 (K; 11.8 in two rounds of 32 x 128), 300 x 8192 x 2048
+// 12.6 / 14.3 (80 x 160, four rows of tiles) and 260 x 8192 x 2048 12.1 / 12.8 (128 x 128, three).
 const ThinTile *thin_pick(const GemmParams &p, bool silu, int cus) {
     const ThinTile *best = nullptr;
-    long long best_bytes = 1250 * 1000 + 1;
+    long long best_bytes = 0;
     if (p.M > 384) return nullptr;
     for (const ThinTile &t : kThinTiles) {
-        if (silu && t.silu == nullptr) continue;
-        if (p.K % (kSub * t.wk) != 0) continue;
+        if ((silu ? t.silu : t.scale) == nullptr || p.K % (kSub * t.wk) != 0) continue;
         const long long bn = silu ? t.bn / 2 : t.bn, nout = silu ? p.N / 2 : p.N;
-        if (((p.M + t.bm - 1) / t.bm) * ((nout + bn - 1) / bn) > cus) continue;
+        const long long rows = (p.M + t.bm - 1) / t.bm, tiles = rows * ((nout + bn - 1) / bn);
+        const bool large = silu && t.bm + t.bn >= 240;
+        if (large && (p.K < (rows > 2 ? 2560 : 2048) || (t.scale == nullptr && rows > 2))) continue;
+        const bool two = large && 4 * tiles >= 7 * cus && tiles <= 2 * cus;
+        if (tiles > cus && !two) continue;
         const long long bytes = (long long)((p.M < t.bm ? p.M : t.bm) + t.bn) * p.K;
-        if (bytes < best_bytes) {
+        if (bytes > 1250 * 1000) continue;
+        if (best == nullptr || bytes * (two ? 2 : 1) < best_bytes) {
             best = &t;
-            best_bytes = bytes;
+            best_bytes = bytes * (two ? 2 : 1);
         }
     }
     return best;

@@ -255,8 +255,9 @@ def mm_i8(qx, sx, qw, sw, bias=None, out_dtype=torch.bfloat16, residual=None, ep
     ``split=True`` gives the kernel a per-stream workspace (``gemm_workspace``; ``split="auto"``: the one
     ``_auto_workspace`` allows, the choice of QLinear's GEMMs) for schedules that split
     tiles along K, with exact int32 partial sums and so the same bits as without it: for 16-bit outputs
-    with K >= 8192 whose output fits at most CUs / 3 tiles of 128 x 160 (128 x 256 for 'silu_mul') -- a
-    short request's down projection -- every tile in K / 2560 parts; for int32 / fp32 outputs a partial
+    with K >= 8192 whose output fits at most CUs / 3 tiles of 128 x 160 (128 x 256 for 'silu_mul') and that no
+    small tile covers in one round (M up to 384 mostly is; that schedule needs no workspace) -- a 512-token
+    request's down projection -- every tile in K / 2560 parts; for int32 / fp32 outputs a partial
     last round of at most CUs / 4 tiles of 256 x 256 over four workgroups each when K >= 8192 and
     M <= 256 (the default schedule runs such a round as 128 x 128 quarter tiles).  ``requant=True``
     returns the per-token int8 quantization (q, s) of the

@@ -625,6 +625,9 @@ def test_gemm_small_m_split_bit_exact(gpu, m, n, k, epi):
     (20, 640, 512, "silu_mul"),         # 16 x 32: 16 gate and 16 up rows
     (33, 3200, 1024, "silu_mul"),       # 32 x 32, ragged rows
     (300, 4224, 256, "silu_mul"),       # 64 x 64, one slab, a last tile past the output
+    (131, 19456, 2048, "silu_mul"),     # 80 x 160, the second row tile 51 rows, 80 outputs a tile
+    (192, 19456, 2048, "silu_mul"),     # 96 x 192, the last tile 32 of 96 outputs wide
+    (300, 19456, 2560, "silu_mul"),     # 128 x 128 in two rounds
 ])
 def test_gemm_few_rows_bit_exact(gpu, m, n, k, epi):
     """Up to 384 rows: one round of small tiles whose waves split K (int32 sums, exact in any order).  Bit-exact
