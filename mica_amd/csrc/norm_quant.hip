@@ -463,18 +463,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
 // row held in registers from its absmax to its quantizer.  Same arithmetic, same bits: the row
 // (+ residual, rounded to bf16), the norm (x * rstd) * (offset + w) rounded to bf16, t = x * inv in
 // fp32, s = max(absmax(t), 1e-8) / 127, q from the guarded quotient t / s.
-#ifndef MICA_SMOOTH_THREADS
-#define MICA_SMOOTH_THREADS 1024
-#endif
-constexpr int kSmoothThreads = MICA_SMOOTH_THREADS;  // a whole CU's 16 rows share one copy of the factors
+// A workgroup's rows (4, 8 or 16: launch_smooth_one_rnd) share one copy of the factors.
 // SMOOTH = false: the same kernel for unsmoothed outputs, whose int8 rows are then all equal: the
 // row is quantized once (the one-FMA half-even quantizer of common.h, exact for bf16 rows) and
 // stored to each output.
-template <int NCH, bool NORM, int NOUT, int RND, bool SMOOTH = true>
-__global__ __launch_bounds__(kSmoothThreads) __attribute__((amdgpu_waves_per_eu(4))) void smooth_one_kernel(RowParams p) {
+template <int NCH, bool NORM, int NOUT, int RND, bool SMOOTH, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS / 256))) void smooth_one_kernel(RowParams p) {
     constexpr int XT = MICA_BF16;
     const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (kSmoothThreads / 64) + (threadIdx.x >> 6);
+    const int row = blockIdx.x * (THREADS / 64) + (threadIdx.x >> 6);
     const bool on = row < p.M;
     const bool has_res = NORM && p.res != nullptr;
     // every output's factors go to LDS: chunk ch = c * 64 + lane of output o at float4
@@ -486,7 +483,7 @@ __global__ __launch_bounds__(kSmoothThreads) __attribute__((amdgpu_waves_per_eu(
     // whole workgroup waiting for its slowest row (which a full __syncthreads() fence would do).
     extern __shared__ float4 inv_sh[];
     constexpr int kSets = SMOOTH ? NOUT : 0;  // factor sets before the norm's multipliers
-    constexpr int kFill = (NCH * 64 + kSmoothThreads - 1) / kSmoothThreads;  // chunks per thread and set
+    constexpr int kFill = (NCH * 64 + THREADS - 1) / THREADS;  // chunks per thread and set
     constexpr int kHalf = (kSets + (NORM ? 1 : 0)) * NCH * 64;
     float4 fin[kSets > 0 ? kSets : 1][kFill][2];
     u32x4 win[NORM ? kFill : 1];
@@ -494,7 +491,7 @@ __global__ __launch_bounds__(kSmoothThreads) __attribute__((amdgpu_waves_per_eu(
     // the compiler's wait before the LDS fill counts only the loads issued after the factors')
 #pragma unroll
     for (int i = 0; i < kFill; ++i) {
-        const int ch = (int)threadIdx.x + i * kSmoothThreads;
+        const int ch = (int)threadIdx.x + i * THREADS;
         const int chc = ch < NCH * 64 ? ch : NCH * 64 - 1;
 #pragma unroll
         for (int o = 0; o < kSets; ++o) {
@@ -520,7 +517,7 @@ __global__ __launch_bounds__(kSmoothThreads) __attribute__((amdgpu_waves_per_eu(
     }
 #pragma unroll
     for (int i = 0; i < kFill; ++i) {
-        const int ch = (int)threadIdx.x + i * kSmoothThreads;
+        const int ch = (int)threadIdx.x + i * THREADS;
         if (ch < NCH * 64) {
 #pragma unroll
             for (int o = 0; o < kSets; ++o) {
@@ -801,9 +798,9 @@ int launch16(const RowParams &p, int xt, bool norm, bool has_inv, hipStream_t st
 
 // smooth_one_kernel when every row of the launch fits the resident waves; -1 otherwise (the caller
 // then takes the grid-stride path)
-template <int NCH, bool NORM, int NOUT, int RND, bool SMOOTH = true>
+template <int NCH, bool NORM, int NOUT, int RND, bool SMOOTH, int THREADS>
 int launch_smooth_one(const RowParams &p, hipStream_t st) {
-    constexpr auto kern = smooth_one_kernel<NCH, NORM, NOUT, RND, SMOOTH>;
+    constexpr auto kern = smooth_one_kernel<NCH, NORM, NOUT, RND, SMOOTH, THREADS>;
     const unsigned lds = (unsigned)(((SMOOTH ? NOUT : 0) + (NORM ? 1 : 0)) * NCH * 64 * 2 * sizeof(float4));
     // the kernel writes exactly NOUT quantized rows and scales per row: never launch it for another
     // output count (a norm-only call has n_out = 0 and no q / s at all)
@@ -814,20 +811,33 @@ int launch_smooth_one(const RowParams &p, hipStream_t st) {
     int per_cu = cached.load(std::memory_order_relaxed);
     if (per_cu <= 0) {
         int occ = 0;
-        per_cu = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, kSmoothThreads, lds) == hipSuccess && occ > 0 ? occ : 1;
+        per_cu = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, THREADS, lds) == hipSuccess && occ > 0 ? occ : 1;
         cached.store(per_cu, std::memory_order_relaxed);
     }
-    constexpr int kRows = kSmoothThreads / 64;
+    constexpr int kRows = THREADS / 64;
     const long long blocks = ((long long)p.M + kRows - 1) / kRows;
     if (blocks > (long long)cu_count_of_current_device() * per_cu) return -1;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kSmoothThreads), lds, st, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(THREADS), lds, st, p);
     return mica_err(hipGetLastError());
 }
 
+template <int NCH, bool NORM, int NOUT, bool SMOOTH, int THREADS>
+int launch_smooth_one_even(const RowParams &p, hipStream_t st) {
+    if (p.rounding == MICA_ROUND_EVEN) return launch_smooth_one<NCH, NORM, NOUT, MICA_ROUND_EVEN, SMOOTH, THREADS>(p, st);
+    return launch_smooth_one<NCH, NORM, NOUT, MICA_ROUND_AWAY, SMOOTH, THREADS>(p, st);
+}
+
+// The smallest workgroup with which the rows take no more than one of them per CU.  The kernel is a chain of
+// latencies (factors, barrier, row, reductions), and rows that share a SIMD also share its VALU, so up to 4 rows per
+// CU want a SIMD each.  K = 2560, us, 16 rows to a workgroup / this rule, at 16, 333, 1024 and 2048 rows: norm 4.69,
+// 4.90, 5.10, 5.31 / 3.48, 3.67, 3.83, 4.14; norm with three smoothed outputs 9.19, 9.97, 10.51, 10.82 / 5.93, 6.56,
+// 6.93, 8.08; quantizer alone, smoothed, 4.11, 4.49, 4.76, 5.02 / 3.27, 3.48, 3.80, 4.21.
 template <int NCH, bool NORM, int NOUT, bool SMOOTH = true>
 int launch_smooth_one_rnd(const RowParams &p, hipStream_t st) {
-    if (p.rounding == MICA_ROUND_EVEN) return launch_smooth_one<NCH, NORM, NOUT, MICA_ROUND_EVEN, SMOOTH>(p, st);
-    return launch_smooth_one<NCH, NORM, NOUT, MICA_ROUND_AWAY, SMOOTH>(p, st);
+    const int cus = cu_count_of_current_device();
+    if (p.M <= cus * 4) return launch_smooth_one_even<NCH, NORM, NOUT, SMOOTH, 256>(p, st);
+    if (p.M <= cus * 8) return launch_smooth_one_even<NCH, NORM, NOUT, SMOOTH, 512>(p, st);
+    return launch_smooth_one_even<NCH, NORM, NOUT, SMOOTH, 1024>(p, st);
 }
 
 // bf16 rows of exactly NCH * 512 elements (the hot widths): no masks, rounding fixed at compile time

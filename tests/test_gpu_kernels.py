@@ -197,6 +197,10 @@ def test_rmsnorm_quant_multi_consumers(gpu, T, K, n):
     (4096, 2, False, "even"),   # gate / up
     (333, 3, True, "away"),
     (5, 1, True, "even"),       # fewer rows than waves in a workgroup
+    (1024, 3, True, "even"),    # four rows for every CU: the last of the small workgroups
+    (1025, 2, False, "even"),   # the first of the middle ones
+    (2049, 3, False, "even"),   # the first of the large
+    (1, 2, False, "away"),
     (20000, 3, True, "even"),   # more rows than resident waves: the grid-stride kernel
 ])
 def test_rmsnorm_quant_all_consumers_smoothed(gpu, T, n, res, rounding):
