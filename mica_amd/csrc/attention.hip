@@ -23,7 +23,8 @@
 // Data movement: Q fragments stay in registers for the whole workgroup.  K tiles arrive by LDS DMA
 // (buffer_load ... lds), 16-byte chunks XOR-swizzled by row so the operand reads are conflict-free;
 // V^T tiles are DMA'd from an image that v_transpose_kernel writes beforehand in exactly the LDS
-// layout.  Two LDS stages: the DMA of tile j + 1 overlaps the MFMAs of tile j.
+// layout.  Two LDS stages: the DMA of tile j + 1 overlaps the MFMAs of tile j; small grids over long keys take
+// a pipelined schedule over kPSt stages instead (PIPE below).
 //
 // Optionally (mica_attention_fwd_rope) the new rows' q / k head RMSNorm and rotary embedding of the
 // attention layers are folded in: each query as its fragments are loaded (the head's halves are a lane

@@ -5,7 +5,7 @@
 // (BM + BN) rows x K bytes at 40 .. 55 bytes per ns and CU (80 with the weights in the last-level cache), and the
 // 128-row and larger tiles of the other kernels leave most CUs idle there (128 x 2560 x 9728: 16 tiles of
 // 128 x 160).  So tiles are as small as one round allows (thin_pick), and where such a tile has fewer fragments
-// than waves, WK of the 8 waves take their own 128 bytes of every slab and the int32 partial sums meet in LDS at
+// than waves, WK of the 4 to 8 waves take their own 128 bytes of every slab and the int32 partial sums meet in LDS at
 // the end (exact in any order: same bits as every other schedule; no workspace, no second workgroup).  NS slabs
 // are in flight per workgroup, up to 144 KiB.
 // Measured on MI355X, weights cold in the caches (24 copies in turn), us, before -> this kernel:
@@ -14,7 +14,7 @@
 //   2560 x 4096 + residual   13.0 ->  4.4   13.3 ->  5.7   14.2 ->  7.4   14.4 ->  9.3
 //   6144 x 2560              19.5 ->  5.9   19.8 ->  8.6   23.6 -> 10.3   21.6 -> 13.2
 //   12352 x 2560             20.1 ->  8.6   20.7 -> 11.8   24.5 -> 15.3   23.3 -> 19.2
-//   19456 x 2560 SiLU        15.3 -> 14.0   17.8 -> 16.1   19.9 -> 19.4   (29.7 -> 29.8 at 224: not taken)
+//   19456 x 2560 SiLU        15.3 -> 14.0   17.8 -> 16.1   19.9 -> 19.4   (29.7: no tile at 193 .. 256 rows)
 // Tried without gain: fragments loaded straight to registers (16 rows x 64 bytes per load: 64 clocks each in
 // the address unit, 16 bytes per clock), a wave that touches the weights ahead of the DMA (they are already as
 // deep in flight as the feed takes them), and a different K start per tile.
