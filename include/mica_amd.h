@@ -311,6 +311,10 @@ int mica_attention_fwd_prefix(const void *q, long long sbq, long long shq, long 
  * sequences' own images for Sk - Pk keys, the split states as above; -1 for an invalid argument */
 long long mica_attention_prefix_workspace_bytes(int B, int Sq, int Sk, int Pk, int HQ, int HK, int key_splits);
 
+/* 1 when an unsplit attention launch of these sizes (any entry point; Sk counts a prefix's keys) runs the pipelined
+ * schedule on a device of `cus` compute units, 0 when two workgroups per CU, -1 for invalid sizes; same bits either way */
+int mica_attention_pipelined(int B, int Sq, int Sk, int HK, int cus);
+
 /*
  * mica_attention_fwd_prefix (kv_len NULL; Pk = 0: no prefix) with the new rows' q / k head norm and rotary
  * embedding folded in: the attention layers' q_norm / k_norm and apply_rotary_pos_emb before the attention

@@ -24,7 +24,7 @@
 // (buffer_load ... lds), 16-byte chunks XOR-swizzled by row so the operand reads are conflict-free;
 // V^T tiles are DMA'd from an image that v_transpose_kernel writes beforehand in exactly the LDS
 // layout.  Two LDS stages: the DMA of tile j + 1 overlaps the MFMAs of tile j; small grids over long keys take
-// a pipelined schedule over kPSt stages instead (PIPE below).
+// a pipelined schedule over kPSt stages instead (PIPE; pipelined() below has the rule).
 //
 // Optionally (mica_attention_fwd_rope) the new rows' q / k head RMSNorm and rotary embedding of the
 // attention layers are folded in: each query as its fragments are loaded (the head's halves are a lane
@@ -64,14 +64,6 @@ constexpr int kPSt = 4;                  // the pipelined schedule's: one read, 
 template <bool PIPE>
 constexpr int kFaSmem = (PIPE ? kPSt : kNSt) * kStage;
 constexpr int kMaxKeySplits = 64;
-// The pipelined schedule serves grids of at most kPipeBlocks workgroups (2 per CU) whose blocks walk at least
-// kPipeKeys keys: there a wave's chain of tiles is what takes the time.  Measured on MI355X (us, two workgroups per
-// CU / pipelined): 1 x 2048 78.2 / 73.5, 1 x 3000 118.1 / 105.9, 4 x 700 42.7 / 40.1, 8 x 240 after 6912 keys 267 / 248,
-// 8 x 64 after 6912 220 / 193; shorter or fuller grids lose by its longer prologue and its one workgroup per CU:
-// 8 x 256 21.9 / 23.7, 8 x 512 39.0 / 45.8, 1 x 256 19.4 / 20.7, 4 x 1500 (752 workgroups) 95.8 / 114.7.
-constexpr int kPipeBlocks = 512;
-constexpr int kPipeKeys = 640;
-
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
@@ -251,7 +243,7 @@ __global__ __launch_bounds__(256) void v_transpose_kernel(FaParams p) {
     }
 }
 
-// PIPE: the schedule of small grids over long keys (kPipeBlocks), one workgroup per CU and one wave per SIMD;
+// PIPE: the schedule of small grids over long keys (pipelined()), one workgroup per CU and one wave per SIMD;
 // otherwise two workgroups per CU, whose waves fill each other's gaps.  Same bits.
 template <bool SPLIT, bool PIPE>
 __global__ __launch_bounds__(kFaThreads, PIPE ? 1 : 2) void fa_fwd_kernel(FaParams p) {
@@ -779,6 +771,31 @@ extern "C" long long mica_attention_split_workspace_bytes(int B, int Sq, int Sk,
 
 namespace {
 
+// Whether an unsplit launch runs the pipelined schedule (one workgroup per CU), on a device of `cus` CUs.  A launch
+// that gives no CU a second workgroup does from 640 keys on: there a block's chain of tiles is what takes the time.
+// Past that the other schedule runs two workgroups of a CU side by side, this one the second behind the first.  The
+// longest blocks are dispatched first, so the second round lasts about twice the tiles `lc` of the block of rank `cus`
+// plus a prologue worth 11 tiles.  That is free where it ends before the longest block's `lmax` tiles do (causal
+// blocks without much of a common past), and the more CUs hold two workgroups, the slower the other schedule is: the
+// line (2.1 - 0.3 workgroups / cus) lc + 11 <= lmax.  kv_len does not move it: Sk bounds the counts, and fewer keys
+// take the same number of tiles off both sides.
+// Measured on MI355X over 302 grids of 257 to 512 workgroups: the line's choice is nowhere more than 1 % behind the
+// other one.  Two workgroups per CU / pipelined, us, the chosen one in brackets:
+//   one round     1 x 2048 75.1 / [69.8], 8 x 64 after 6912 keys 220.8 / [194.9], 8 x 256 after 6912 246.5 / [237.3],
+//                 8 x 256 after 640 44.4 / [44.2]
+//   two rounds    1 x 2176 82.9 / [73.5], 1 x 4096 165.8 / [151.6], 2 x 1408 61.1 / [53.5], 2 x 1280 after 640 83.9 /
+//                 [82.2]; 8 x 288 after 640 [54.7] / 66.3, 8 x 288 after 6912 [329.8] / 408.8, 8 x 512 after 6912
+//                 [428.6] / 465.7, 4 x 1024 [54.9] / 56.6, 100 last rows after 2048 [99.1] / 120.1
+//   short keys    8 x 256 [21.9] / 23.7, 1 x 256 [19.4] / 20.7; three rounds 4 x 1500 [95.8] / 114.7
+bool pipelined(long long B, long long Sq, long long Sk, long long HK, long long cus) {
+    const long long per = B * HK, ntq = (Sq + kBQ - 1) / kBQ, wgs = per * ntq;
+    if (wgs == 0 || Sk < 640 || wgs > 2 * cus) return false;
+    if (wgs <= cus) return true;
+    const long long rank = cus / per, q = ntq - 1 - rank, ntk = (Sk + kBK - 1) / kBK;
+    const long long end = (Sk - Sq + q * kBQ + kBQ - 1) / kBK + 1, lc = end < ntk ? end : ntk;
+    return (21 * cus - 3 * wgs) * lc + 110 * cus <= 10 * cus * ntk;
+}
+
 // kp / vp (optional, Pk > 0 keys, a multiple of 32): a key prefix shared by every sequence, read in
 // place of each sequence's first Pk keys; k / v then hold each sequence's Sk - Pk keys after it.
 int attention_launch(const void *q, long long sbq, long long shq, long long ldq, const void *k, long long sbk,
@@ -868,7 +885,11 @@ int attention_launch(const void *q, long long sbq, long long shq, long long ldq,
         if (rc) return rc;
     }
     if (key_splits == 1) {
-        if ((long long)HK * B * ntiles_q <= kPipeBlocks && Sk >= kPipeKeys)
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            cus = 0;
+        if (pipelined(B, Sq, Sk, HK, cus))
             hipLaunchKernelGGL((fa_fwd_kernel<false, true>), dim3(HK, B, ntiles_q), dim3(kFaThreads), 0, stream_, p);
         else
             hipLaunchKernelGGL((fa_fwd_kernel<false, false>), dim3(HK, B, ntiles_q), dim3(kFaThreads), 0, stream_, p);
@@ -884,6 +905,11 @@ int attention_launch(const void *q, long long sbq, long long shq, long long ldq,
 }
 
 }  // namespace
+
+extern "C" int mica_attention_pipelined(int B, int Sq, int Sk, int HK, int cus) {
+    if (B < 0 || Sq < 0 || Sk < Sq || HK <= 0 || cus < 0) return -1;
+    return pipelined(B, Sq, Sk, HK, cus) ? 1 : 0;
+}
 
 extern "C" int mica_attention_fwd(const void *q, long long sbq, long long shq, long long ldq, const void *k, long long sbk,
                                   long long shk, long long ldk, const void *v, long long sbv, long long shv,

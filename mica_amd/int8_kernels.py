@@ -123,8 +123,8 @@ def preload(device=None) -> int:
     ok, _ = available(device)
     if not ok:
         return 0
-    return sum(1 for name in _lib.SIGNATURES if name not in ("mica_version", "mica_status_name",
-                                                            "mica_device_info"))
+    return sum(1 for name in _lib.SIGNATURES if name not in ("mica_version", "mica_status_name", "mica_device_info",
+                                                            "mica_attention_pipelined"))
 
 
 def _stream(dev) -> int:

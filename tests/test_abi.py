@@ -229,6 +229,25 @@ def test_gdn_chunk_rejects():
     assert lib.mica_gdn_workspace_bytes(8, 2048, 32) == 8 * 32 * 32 * (2 * 64 * 128 * 2 + 64 * 4)
 
 
+@pytest.mark.parametrize("B,Sq,Sk,want", [
+    (8, 256, 7168, 1),     # one workgroup for every CU
+    (1, 32, 640, 1), (1, 32, 639, 0),
+    (8, 257, 7169, 0),     # 288: a second round of blocks as long as the first (329.8 us, pipelined 408.8)
+    (8, 512, 7424, 0), (4, 544, 1184, 0), (8, 500, 700, 0), (100, 1, 2112, 0), (1, 2500, 5000, 0),
+    (1, 2176, 2176, 1),    # 272: the second round's blocks are the shortest (82.9 us, pipelined 73.5)
+    (2, 1408, 1408, 1), (1, 4096, 4096, 1), (2, 1280, 1920, 1), (1, 3072, 4096, 1),
+    (4, 1024, 1024, 0),    # 512, the second round as long as the longest block (54.9 us, pipelined 56.6)
+    (1, 4128, 4128, 0),    # 516: more than two per CU
+])
+def test_attention_schedule_by_rounds(B, Sq, Sk, want):
+    """The pipelined schedule is taken where its one workgroup per CU is not slower than two: on grids of one
+    round, and past that only where the second round's blocks are short beside the longest one."""
+    lib = _lib.load()
+    assert lib.mica_attention_pipelined(B, Sq, Sk, 4, 256) == want
+    assert lib.mica_attention_pipelined(0, 1, 700, 4, 256) == 0
+    assert lib.mica_attention_pipelined(B, Sq, Sk, 4, 0) == 0 and lib.mica_attention_pipelined(B, Sk + 1, Sk, 4, 256) == -1
+
+
 def test_gdn_chunk_gate_rejects():
     lib = _lib.load()
     D = 128
