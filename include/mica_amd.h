@@ -142,6 +142,11 @@ int mica_mm_i8(const int8_t *A, int lda, const int8_t *B, int ldb, const float *
 /* bytes of GEMM workspace for `device` (its CU count x 512 KiB + 4 KiB), or -(hipError_t) */
 long long mica_mm_i8_workspace_bytes(int device);
 
+/* 1 when a 16-bit-output mica_mm_i8 of these sizes on a device of `cus` compute units runs as one round of small tiles
+ * (no workspace needed), tile[0 .. 2] then being the tile's rows, its weight rows and the waves that share K; 0 when
+ * another schedule runs, -1 for invalid sizes.  (Operands that reach 2^31 bytes a tile past their last row never do.) */
+int mica_mm_i8_few_rows_tile(int M, int N, int K, int epilogue, int cus, int *tile);
+
 /*
  * mica_mm_i8 for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same

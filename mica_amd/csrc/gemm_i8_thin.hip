@@ -334,26 +334,44 @@ const ThinTile kThinTiles[] = {
 
 // The tile that streams the fewest bytes per CU among those that cover the output in one round (128 x 128 with SiLU:
 // or in two, the second three quarters full) and whose waves' K shares divide K; none past 384 rows or 1.25 MB a
-// round; with SiLU, tiles of 128 x 128 and more want K >= 2048 (2560 past two rows of tiles) and the two of SiLU's own
-// at most two rows of tiles.  Measured against the other kernels (us, cold weights, other / this): 384 x 6144 x 2560
-// 21.5 / 17.8, 384 x 2560 x 9728 46.6 / 24.0, 8192 x 1024 at 40 rows 9.7 / 5.3, at 384 10.8 / 10.1, SiLU x 19456 x 2560
-// at 131 rows 26.3 / 20.2, 192 28.7 / 23.4, 300 38.1 / 30.7 (two rounds); past the lines 512 x 6144 x 2560 16.5 / 18.7
-// (rows), 512 x 2560 x 9728 28.9 / 35 (bytes, 128 x 64 tiles), 384 x 12352 x 2560 19.6 / 33.9 (1.1 rounds), SiLU 224 x
-// 24576 x 4096 42.7 / 47.8 (1.5), 131 x 12288 x 1024 9.0 / 10.3 (K; 11.8 in two rounds of 32 x 128), 300 x 8192 x 2048
-// 12.6 / 14.3 (80 x 160, four rows of tiles) and 260 x 8192 x 2048 12.1 / 12.8 (128 x 128, three).
-const ThinTile *thin_pick(const GemmParams &p, bool silu, int cus) {
+// round.  The large tiles (128 x 128, and SiLU's own 80 x 160 and 96 x 192) have lines of their own:
+//   plain: K >= 1536 (1152 where the kernels of 256-byte K steps don't serve K), and where the AGPR kernel covers the
+//     output in one round of 128 x 160 tiles (gemm_i8.hip) at most 128 rows and K >= 2560;
+//   SiLU: K >= 2048 (2560 past two rows of tiles), and its own two at most two rows of tiles.
+// Measured against what would run instead, the split along K included (us, other / this; cold: 24 copies of the weights
+// in turn, as in a model; warm: the same weights again, which stay in the caches).  Cold: 384 x 6144 x 2560 21.4 /
+// 17.7, 384 x 2560 x 9728 28.8 / 24.2, 8192 x 1024 at 40 rows 9.7 / 5.3, SiLU x 19456 x 2560 at 131 rows 24.9 / 19.1,
+// 192 27.3 / 22.6, 300 37.0 / 29.6 (two rounds).  Past the lines, cold, then warm:
+//   512 x 6144 x 2560 16.5 / 18.7 cold (rows), 512 x 2560 x 9728 28.9 / 35 (bytes, 128 x 64 tiles), 384 x 12352 x 2560
+//   19.6 / 33.9 (1.1 rounds), SiLU 224 x 24576 x 4096 42.7 / 47.8 (1.5);
+//   plain 128 x 128, K: 321 x 6144 x 1024 7.9 / 9.1, 6.7 / 9.1; 256 x 10240 x 1024 8.4 / 9.3, 6.9 / 9.1; 257 x 8192 x
+//   512 6.0 / 7.7, 5.4 / 7.4; on the other side 257 x 8192 x 1536 12.9 / 11.5, 8.3 / 11.1 and 256 x 12288 x 1280 13.0 /
+//   12.1, 8.2 / 10.4 (K = 1280 at 257 x 8192: 9.3 / 10.2);
+//   plain 128 x 128, one AGPR round: 257 x 10240 x 2560 16.3 / 16.3, 12.7 / 15.6; 257 x 9728 x 3584 18.6 / 20.9, 16.4 /
+//   20.3; 128 x 32768 x 2048 18.2 / 19.3, 14.6 / 16.8; on the other side 128 x 19456 x 4096 30.4 / 28.3, 17.9 / 20.5;
+//   SiLU: 131 x 12288 x 1024 9.0 / 10.3 cold (K; 11.8 in two rounds of 32 x 128), 300 x 8192 x 2048 12.6 / 14.3 (80 x
+//   160, four rows of tiles), 260 x 8192 x 2048 12.1 / 12.8 (128 x 128, three).
+// Cold decides: a model's weights are read once a pass.  Inside the lines the tiles of 128 x 128 are up to 20 % faster
+// cold and up to 24 % slower warm (321 x 6144 x 2560 19.8 / 16.4, 11.2 / 14.6): the larger tiles of the other kernels
+// read fewer bytes, this one has more of them in flight.
+const ThinTile *thin_pick(int M, long long N, int K, bool silu, int cus) {
     const ThinTile *best = nullptr;
     long long best_bytes = 0;
-    if (p.M > 384) return nullptr;
+    if (M > 384) return nullptr;
+    const long long nout = silu ? N / 2 : N, rows128 = (M + 127) / 128;
+    const long long tiles256 = (M + 255) / 256 * ((N + 255) / 256);
+    const bool agpr_round = !silu && K % 256 == 0 && nout % 8 == 0 && 4 * tiles256 > cus && 2 * tiles256 <= cus &&
+                            rows128 * ((N + 159) / 160) <= cus;
     for (const ThinTile &t : kThinTiles) {
-        if ((silu ? t.silu : t.scale) == nullptr || p.K % (kSub * t.wk) != 0) continue;
-        const long long bn = silu ? t.bn / 2 : t.bn, nout = silu ? p.N / 2 : p.N;
-        const long long rows = (p.M + t.bm - 1) / t.bm, tiles = rows * ((nout + bn - 1) / bn);
-        const bool large = silu && t.bm + t.bn >= 240;
-        if (large && (p.K < (rows > 2 ? 2560 : 2048) || (t.scale == nullptr && rows > 2))) continue;
-        const bool two = large && 4 * tiles >= 7 * cus && tiles <= 2 * cus;
+        if ((silu ? t.silu : t.scale) == nullptr || K % (kSub * t.wk) != 0) continue;
+        const long long bn = silu ? t.bn / 2 : t.bn;
+        const long long rows = (M + t.bm - 1) / t.bm, tiles = rows * ((nout + bn - 1) / bn);
+        const bool large = t.bm + t.bn >= 240;
+        if (large && silu && (K < (rows > 2 ? 2560 : 2048) || (t.scale == nullptr && rows > 2))) continue;
+        if (large && !silu && (K < (K % 256 == 0 ? 1536 : 1152) || (agpr_round && (M > 128 || K < 2560)))) continue;
+        const bool two = large && silu && 4 * tiles >= 7 * cus && tiles <= 2 * cus;
         if (tiles > cus && !two) continue;
-        const long long bytes = (long long)((p.M < t.bm ? p.M : t.bm) + t.bn) * p.K;
+        const long long bytes = (long long)((M < t.bm ? M : t.bm) + t.bn) * K;
         if (bytes > 1250 * 1000) continue;
         if (best == nullptr || bytes * (two ? 2 : 1) < best_bytes) {
             best = &t;
@@ -365,10 +383,19 @@ const ThinTile *thin_pick(const GemmParams &p, bool silu, int cus) {
 
 }  // namespace
 
+extern "C" int mica_mm_i8_few_rows_tile(int M, int N, int K, int epilogue, int cus, int *tile) {
+    if (M < 0 || N <= 0 || K <= 0 || K % 16 != 0 || cus < 0 || tile == nullptr) return -1;
+    if (epilogue != MICA_EPI_SCALE && (epilogue != MICA_EPI_SILU_MUL || N % 128 != 0)) return -1;
+    const ThinTile *t = M > 0 ? thin_pick(M, N, K, epilogue == MICA_EPI_SILU_MUL, cus) : nullptr;
+    if (t == nullptr) return 0;
+    tile[0] = t->bm, tile[1] = t->bn, tile[2] = t->wk;
+    return 1;
+}
+
 bool mica_gemm::thin_launch(const GemmParams &p, int epilogue, int out_dtype, int cus, bool has_bias, bool has_res,
                             hipStream_t st, int *rc) {
     const bool silu = epilogue == MICA_EPI_SILU_MUL;
-    const ThinTile *t = thin_pick(p, silu, cus);
+    const ThinTile *t = thin_pick(p.M, p.N, p.K, silu, cus);
     if (t == nullptr) return false;
     *rc = (silu ? t->silu : t->scale)(p, out_dtype, has_bias, has_res, st);
     return true;

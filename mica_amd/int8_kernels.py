@@ -124,7 +124,7 @@ def preload(device=None) -> int:
     if not ok:
         return 0
     return sum(1 for name in _lib.SIGNATURES if name not in ("mica_version", "mica_status_name", "mica_device_info",
-                                                            "mica_attention_pipelined"))
+                                                            "mica_attention_pipelined", "mica_mm_i8_few_rows_tile"))
 
 
 def _stream(dev) -> int:

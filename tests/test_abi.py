@@ -229,6 +229,30 @@ def test_gdn_chunk_rejects():
     assert lib.mica_gdn_workspace_bytes(8, 2048, 32) == 8 * 32 * 32 * (2 * 64 * 128 * 2 + 64 * 4)
 
 
+def few_rows_tile(M, N, K, epilogue=0, cus=256):
+    t = (ctypes.c_int * 3)()
+    rc = _lib.load().mica_mm_i8_few_rows_tile(M, N, K, epilogue, cus, t)
+    return tuple(t) if rc == 1 else {0: None}.get(rc, rc)
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    (321, 6144, 1024, None), (256, 10240, 1024, None), (257, 8192, 512, None),  # K too short for 128 x 128
+    (257, 8192, 1280, None), (257, 8192, 1536, (128, 128, 1)), (256, 12288, 1152, (128, 128, 1)),
+    (257, 10240, 2560, None), (384, 9728, 2560, None), (257, 8704, 3584, None),  # one round of 128 x 160 elsewhere
+    (384, 8192, 2560, (128, 128, 1)), (321, 6144, 2560, (128, 128, 1)), (256, 10240, 2560, (128, 128, 1)),
+    (128, 19456, 2048, None), (128, 19456, 2560, (128, 128, 1)), (128, 16384, 2560, (128, 64, 1)),
+    (257, 10248, 2560, None), (257, 10242, 2560, (128, 128, 1)),  # the other round writes whole 16-byte units
+    (385, 2560, 9728, None), (8, 2560, 9728, (16, 16, 4)), (8, 2560, 9744, None),
+])
+def test_few_rows_tile_of_plain_gemms(M, N, K, want):
+    assert few_rows_tile(M, N, K) == want
+
+
+def test_few_rows_tile_rejects():
+    assert few_rows_tile(8, 64, 40) == -1 and few_rows_tile(8, 64, 64, 2) == -1 and few_rows_tile(8, 192, 128, 1) == -1
+    assert few_rows_tile(0, 64, 128) is None and few_rows_tile(8, 64, 128, 0, 0) is None
+
+
 @pytest.mark.parametrize("B,Sq,Sk,want", [
     (8, 256, 7168, 1),     # one workgroup for every CU
     (1, 32, 640, 1), (1, 32, 639, 0),
