@@ -337,7 +337,8 @@ const ThinTile kThinTiles[] = {
 // round.  The large tiles (128 x 128, and SiLU's own 80 x 160 and 96 x 192) have lines of their own:
 //   plain: K >= 1536 (1152 where the kernels of 256-byte K steps don't serve K), and where the AGPR kernel covers the
 //     output in one round of 128 x 160 tiles (gemm_i8.hip) at most 128 rows and K >= 2560;
-//   SiLU: K >= 2048 (2560 past two rows of tiles), and its own two at most two rows of tiles.
+//   SiLU: K >= 2048 (2560 past two rows of tiles), its own two at most two rows of tiles, and where the AGPR kernel
+//     covers the output in one round of 128 x 128 tiles at most 128 rows.
 // Measured against what would run instead, the split along K included (us, other / this; cold: 24 copies of the weights
 // in turn, as in a model; warm: the same weights again, which stay in the caches).  Cold: 384 x 6144 x 2560 21.4 /
 // 17.7, 384 x 2560 x 9728 28.8 / 24.2, 8192 x 1024 at 40 rows 9.7 / 5.3, SiLU x 19456 x 2560 at 131 rows 24.9 / 19.1,
@@ -349,8 +350,10 @@ const ThinTile kThinTiles[] = {
 //   12.1, 8.2 / 10.4 (K = 1280 at 257 x 8192: 9.3 / 10.2);
 //   plain 128 x 128, one AGPR round: 257 x 10240 x 2560 16.3 / 16.3, 12.7 / 15.6; 257 x 9728 x 3584 18.6 / 20.9, 16.4 /
 //   20.3; 128 x 32768 x 2048 18.2 / 19.3, 14.6 / 16.8; on the other side 128 x 19456 x 4096 30.4 / 28.3, 17.9 / 20.5;
-//   SiLU: 131 x 12288 x 1024 9.0 / 10.3 cold (K; 11.8 in two rounds of 32 x 128), 300 x 8192 x 2048 12.6 / 14.3 (80 x
-//   160, four rows of tiles), 260 x 8192 x 2048 12.1 / 12.8 (128 x 128, three).
+//   SiLU: 131 x 12288 x 1024 9.0 / 10.3 cold (K; 11.8 in two rounds of 32 x 128); one AGPR round: 129 x 16384 x 2304
+//   13.6 / 15.5, 12.4 / 14.3; 160 x 12288 x 2560 15.6 / 18.7, 12.3 / 15.2; 384 x 6144 x 3072 19.0 / 18.2, 12.5 / 15.6
+//   (at most 128 rows: 128 x 19456 x 2560 19.8 / 19.2, 13.6 / 15.9).  K = 2048 to 2432 in two rounds past two rows of
+//   tiles, which the line leaves out, would gain: 257 x 19456 x 2304 33.8 / 27.1.
 // Cold decides: a model's weights are read once a pass.  Inside the lines the tiles of 128 x 128 are up to 20 % faster
 // cold and up to 24 % slower warm (321 x 6144 x 2560 19.8 / 16.4, 11.2 / 14.6): the larger tiles of the other kernels
 // read fewer bytes, this one has more of them in flight.
@@ -360,14 +363,16 @@ const ThinTile *thin_pick(int M, long long N, int K, bool silu, int cus) {
     if (M > 384) return nullptr;
     const long long nout = silu ? N / 2 : N, rows128 = (M + 127) / 128;
     const long long tiles256 = (M + 255) / 256 * ((N + 255) / 256);
-    const bool agpr_round = !silu && K % 256 == 0 && nout % 8 == 0 && 4 * tiles256 > cus && 2 * tiles256 <= cus &&
-                            rows128 * ((N + 159) / 160) <= cus;
+    const bool agpr_round = K % 256 == 0 && nout % 8 == 0 &&
+                            (silu ? rows128 * (N / 128) <= cus
+                                  : 4 * tiles256 > cus && 2 * tiles256 <= cus && rows128 * ((N + 159) / 160) <= cus);
     for (const ThinTile &t : kThinTiles) {
         if ((silu ? t.silu : t.scale) == nullptr || K % (kSub * t.wk) != 0) continue;
         const long long bn = silu ? t.bn / 2 : t.bn;
         const long long rows = (M + t.bm - 1) / t.bm, tiles = rows * ((nout + bn - 1) / bn);
         const bool large = t.bm + t.bn >= 240;
-        if (large && silu && (K < (rows > 2 ? 2560 : 2048) || (t.scale == nullptr && rows > 2))) continue;
+        if (large && silu && (K < (rows > 2 ? 2560 : 2048) || (t.scale == nullptr && rows > 2) || (agpr_round && M > 128)))
+            continue;
         if (large && !silu && (K < (K % 256 == 0 ? 1536 : 1152) || (agpr_round && (M > 128 || K < 2560)))) continue;
         const bool two = large && silu && 4 * tiles >= 7 * cus && tiles <= 2 * cus;
         if (tiles > cus && !two) continue;

@@ -248,6 +248,19 @@ def test_few_rows_tile_of_plain_gemms(M, N, K, want):
     assert few_rows_tile(M, N, K) == want
 
 
+@pytest.mark.parametrize("M,N,K,want", [
+    # one round of 128 x 128 tiles of the other kernel
+    (129, 16384, 2304, None), (160, 12288, 2560, None), (192, 14336, 4096, None), (384, 6144, 3072, None),
+    (131, 16512, 2560, (80, 160, 1)),    # 258 of them: more than one round
+    (129, 16384, 2176, (80, 160, 1)),    # K no multiple of 256: not a K of that kernel
+    (128, 19456, 2560, (80, 160, 1)), (100, 16384, 2560, (128, 64, 1)), (192, 8192, 2560, (128, 64, 1)),
+    (131, 19456, 2560, (80, 160, 1)), (192, 19456, 2560, (96, 192, 1)), (300, 19456, 2560, (128, 128, 1)),
+    (300, 19456, 2304, None),
+])
+def test_few_rows_tile_of_silu_gemms(M, N, K, want):
+    assert few_rows_tile(M, N, K, 1) == want
+
+
 def test_few_rows_tile_rejects():
     assert few_rows_tile(8, 64, 40) == -1 and few_rows_tile(8, 64, 64, 2) == -1 and few_rows_tile(8, 192, 128, 1) == -1
     assert few_rows_tile(0, 64, 128) is None and few_rows_tile(8, 64, 128, 0, 0) is None
