@@ -3,7 +3,8 @@ launch path over it (binding/native.cpp, _native.so).
 
 The library is loaded after torch, so it binds to the HIP runtime torch already loaded (same soname)
 and the stream handles torch hands out are valid in it.  A missing library is an error, never a
-silent fallback: build it with ``python -m mica_amd.build``.
+silent fallback: build it with ``python -m mica_amd.build``.  Without the launch path calls go through Python,
+with a warning.
 """
 from __future__ import annotations
 
@@ -12,10 +13,13 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 from pathlib import Path
 
 LIB_NAME = "libmica_amd.so"
 ENV_DIR = "MICA_AMD_LIB_DIR"
+# always the package's own (its functions' arguments are those the package's Python files pass), whatever ENV_DIR names
+NATIVE_PATH = Path(__file__).resolve().parent / "_native.so"
 
 # dtype codes (mica_amd.h)
 BF16, FP16, FP32, INT8, INT32 = 0, 1, 2, 3, 4
@@ -84,7 +88,7 @@ NATIVE_FNS = ("mica_act_quant", "mica_mm_i8", "mica_rmsnorm_quant", "mica_rmsnor
 
 
 class _NotLoaded:
-    """Stands for the native launch path until load(): every function declines the call."""
+    """Stands for the native launch path until load(), or where it does not load: every function declines the call."""
 
     def __getattr__(self, name):
         return lambda *args: None
@@ -104,12 +108,16 @@ def lib_path() -> Path:
 
 
 def _load_native(lib):
-    path = Path(__file__).resolve().parent / "_native.so"
-    if not path.is_file():
-        raise RuntimeError(f"{path} is not built; run `python -m mica_amd.build`")
-    loader = importlib.machinery.ExtensionFileLoader("mica_amd._native", str(path))
-    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("mica_amd._native", loader))
-    loader.exec_module(mod)
+    """The launch path over `lib`, or its stand-in when the module is missing or does not load under this torch and
+    Python: the Python path serves every call, so that is a warning about host time and no error."""
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("mica_amd._native", str(NATIVE_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("mica_amd._native", loader))
+        loader.exec_module(mod)
+    except (ImportError, OSError) as exc:
+        warnings.warn(f"mica_amd: no native launch path ({exc}); calls take 10 to 100 us more host time each. Rebuild "
+                      "with `python -m mica_amd.build`", RuntimeWarning, stacklevel=3)
+        return _NotLoaded()
     mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in NATIVE_FNS})
     return mod
 

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from mica_amd import fused_kernels, int8_kernels, int8_runtime
+from mica_amd import _lib, fused_kernels, int8_kernels, int8_runtime
 from mica_amd.readout import LabelReadout
 from oracle import w8a8 as O
 
@@ -14,6 +14,20 @@ def lenient(monkeypatch):
     monkeypatch.setattr(int8_kernels, "STRICT", False)
     int8_kernels.STATS["fallback"].clear()
     return int8_kernels.STATS
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared object"])
+def test_a_missing_or_broken_launch_path_leaves_the_python_path(monkeypatch, tmp_path, content):
+    """load() goes on with the declining stand-in, and says so: libmica_amd.so alone serves every call."""
+    path = tmp_path / "_native.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_lib, "NATIVE_PATH", path)
+    monkeypatch.setattr(_lib, "_LIB", None)
+    monkeypatch.setattr(_lib, "FAST", None)
+    with pytest.warns(RuntimeWarning, match="no native launch path"):
+        lib = _lib.load()
+    assert lib.mica_version() == 1 and _lib.FAST.act_quant(None, None, 0) is None
 
 
 def test_cpu_inputs_miss_like_the_reference(lenient):
