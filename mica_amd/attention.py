@@ -61,7 +61,9 @@ def attention_fwd(q, k, v, q_layout: str, scale: float | None = None, key_splits
     ``fused_kernels.rope_inplace`` / ``head_norm_rope`` treat it; q as the kernel loads it, unchanged in
     memory.  The result equals those passes over q and k followed by the plain call, bit for bit."""
     if kv_len is None and rope is None and head_norm is None and key_splits == 1 and q_layout in ("bshd", "bhsd"):
-        kp, vp = prefix if prefix is not None else (None, None)
+        kp = vp = None
+        if prefix is not None:
+            kp, vp = prefix = tuple(prefix)    # (any iterable of two: the path below reads it again)
         r = _lib.FAST.attention(q, k, v, q_layout == "bshd",
                                 1.0 / math.sqrt(HEAD_DIM) if scale is None else float(scale), kp, vp)
         if r is not None:

@@ -121,6 +121,17 @@ def test_native_path_equals_python_path(gpu, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_prefix_from_an_iterator_survives_a_declined_call(gpu):
+    """The native path declines [1, P, heads, 256] prefix views; the Python path after it still finds them."""
+    g = torch.Generator(device=gpu).manual_seed(5)
+    qkv = torch.randn(2, 40, 24, 256, generator=g, device=gpu).to(BF)
+    q, k, v = qkv.split((16, 4, 4), dim=2)
+    pre = torch.randn(2, 64, 4, 256, generator=g, device=gpu).to(BF)
+    want = causal_gqa_attention(q, k, v, prefix=(pre[0], pre[1]))
+    assert torch.equal(causal_gqa_attention(q, k, v, prefix=iter((pre[:1], pre[1:]))), want)
+
+
+@pytest.mark.gpu
 def test_native_path_leaves_watched_calls_to_python(gpu):
     """A dispatch mode, vmap or a tensor subclass: the native path declines, whatever Python then does."""
     x = torch.ones(4, 512, device=gpu, dtype=BF)
