@@ -121,6 +121,71 @@ def test_native_path_equals_python_path(gpu, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_native_path_equals_python_path_on_a_side_stream(gpu, monkeypatch):
+    """As above on a stream of its own, which the inputs were not made on: launches, outputs and the GEMM's workspace
+    are that stream's."""
+    monkeypatch.setattr(int8_kernels, "STRICT", False)
+    fns = forms(gpu)
+    side = torch.cuda.Stream(gpu)
+    side.wait_stream(torch.cuda.current_stream(gpu))
+    for name, fn in fns.items():
+        with torch.cuda.stream(side):
+            a, b = outcome(fn, True), outcome(fn, False)
+        side.synchronize()
+        assert a[1:] == b[1:], (name, a[1:], b[1:])
+        for s, t in zip(flat(a[0]), flat(b[0])):
+            assert (s is None and t is None) or torch.equal(s, t), name
+    torch.cuda.current_stream(gpu).wait_stream(side)
+
+
+@pytest.mark.gpu
+def test_native_path_equals_python_path_in_a_captured_graph(gpu):
+    """One graph of a chain of calls on the native path, one on the Python path: every replay, with eager work between,
+    gives the eager bits, after the inputs changed in place too."""
+    g = torch.Generator(device=gpu).manual_seed(11)
+    x = torch.randn(40, 2560, generator=g, device=gpu).to(BF)
+    w = torch.randn(2560, generator=g, device=gpu).to(BF)
+    qw = torch.randint(-127, 128, (6144, 2560), generator=g, device=gpu, dtype=torch.int8)
+    sw = torch.rand(6144, generator=g, device=gpu) * 1e-2
+    dw = torch.randint(-127, 128, (2560, 9728), generator=g, device=gpu, dtype=torch.int8)
+    ds = torch.rand(2560, generator=g, device=gpu) * 1e-2
+    h = torch.randn(440, 9728, generator=g, device=gpu).to(BF)
+
+    def chain():
+        (q, s), = fused_kernels.rms_norm_quant_multi(x, w, 1e-6, [None])
+        y = int8_kernels.mm_i8(q, s, qw, sw, split="auto").view(1, 40, 24, 256)
+        o = causal_gqa_attention(*y.split((16, 4, 4), dim=2))
+        # 440 rows: the split along K, through the capturing stream's workspace
+        return o, int8_kernels.mm_i8(*int8_kernels.act_quant(h), dw, ds, split="auto")
+
+    stream = torch.cuda.Stream(gpu)
+    runs = []
+    keep = _lib.FAST
+    try:
+        for fast in (True, False):
+            _lib.FAST = keep if fast else _lib._NotLoaded()
+            stream.wait_stream(torch.cuda.current_stream(gpu))
+            with torch.cuda.stream(stream):
+                chain()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=stream):
+                    out = chain()
+            runs.append((graph, out))
+    finally:
+        _lib.FAST = keep
+    for i in range(4):
+        if i == 2:
+            x.mul_(-0.5)
+            h.mul_(0.25)
+        want = chain()
+        for graph, out in runs:
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(out, want):
+                assert torch.equal(a, b), i
+
+
+@pytest.mark.gpu
 def test_prefix_from_an_iterator_survives_a_declined_call(gpu):
     """The native path declines [1, P, heads, 256] prefix views; the Python path after it still finds them."""
     g = torch.Generator(device=gpu).manual_seed(5)
