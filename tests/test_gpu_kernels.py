@@ -1027,17 +1027,24 @@ def test_attention_split_keys_matches_oracle(gpu, B, Sq, Sk, HK, splits):
     assert w_split <= 2.0 * w_one + 1e-3
 
 
-@pytest.mark.parametrize("B,S,P", [
-    (5, 1024, 0),    # 640 workgroups together, 128 alone: the two schedules
-    (17, 250, 640),  # 544 / 32, queries past the last tile's end, the diagonal across two tiles of a prefix's end
-    (16, 263, 1088), # 576 / 36, 9 query blocks, the last 7 rows long
+@pytest.mark.parametrize("B,S,P,Sq", [
+    (5, 1024, 0, 1024),    # 640 workgroups together, 128 alone: the two schedules
+    (17, 250, 640, 250),   # 544 / 32, queries past the last tile's end, the diagonal across two tiles of a prefix's end
+    (16, 263, 1088, 263),  # 576 / 36, 9 query blocks, the last 7 rows long
+    (8, 257, 640, 257),    # 288 / 36: a second round as long as the first
+    (70, 90, 640, 1),      # 280 / 4, one query each at kv_len: in every tile of the new keys, at its ends and inside
+    (66, 690, 0, 40),      # 528 / 8, kv_len without a prefix, two query blocks
 ])
-def test_attention_schedules_agree_bit_for_bit(gpu, B, S, P):
+def test_attention_schedules_agree_bit_for_bit(gpu, B, S, P, Sq):
     """Few workgroups over long keys run the pipelined schedule, more of them the other: the sequences of a batch run
     together and alone must agree in every bit (the same arithmetic per query)."""
+    from mica_amd import _lib
     from mica_amd.attention import causal_gqa_attention
 
-    note(f"attention schedules B={B} S={S} P={P}")
+    note(f"attention schedules B={B} S={S} P={P} Sq={Sq}")
+    cus = _lib.device_info(gpu.index)["cu_count"]
+    took = [_lib.load().mica_attention_pipelined(b, Sq, P + S, 4, cus) for b in (B, 1)]
+    assert took == [0, 1], "the batch and a sequence alone no longer run different schedules"
     g = torch.Generator(device=gpu).manual_seed(B * S + P)
     qkv = torch.randn(B, S, 24, 256, generator=g, device=gpu).to(torch.bfloat16)
     qkv[:, S // 2:] *= 3          # maxima that grow late: the rescale runs beyond the first tiles
@@ -1046,9 +1053,14 @@ def test_attention_schedules_agree_bit_for_bit(gpu, B, S, P):
     if P:
         kv = torch.randn(2, P, 4, 256, generator=g, device=gpu).to(torch.bfloat16)
         pre = (kv[0], kv[1])
-    together = causal_gqa_attention(q, k, v, prefix=pre)
+    kv_len, one = None, lambda b: None
+    if Sq < S:
+        q = q[:, S - Sq:]
+        kv_len = torch.tensor([P + S - (b * 7) % (S - Sq + 1) for b in range(B)], dtype=torch.int32, device=gpu)
+        one = lambda b: kv_len[b:b + 1].clone()  # noqa: E731
+    together = causal_gqa_attention(q, k, v, prefix=pre, kv_len=kv_len)
     for b in range(B):
-        alone = causal_gqa_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], prefix=pre)
+        alone = causal_gqa_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], prefix=pre, kv_len=one(b))
         assert torch.equal(alone[0], together[b]), b
 
 
@@ -1058,6 +1070,7 @@ def test_attention_schedules_agree_bit_for_bit(gpu, B, S, P):
     (4, 1024, 64, 64, 1, 5, False),   # split keys over the prefix and the new keys
     (3, 128, 70, 1, 1, 1, True),      # the last-only pass: one query per sequence at kv_len
     (2, 32, 33, 1, 1, 3, True),       # one prefix tile, split, per-sequence key counts
+    (24, 704, 70, 1, 1, 1, True),     # the pipelined schedule: counts from the last new key down to the first
 ])
 def test_attention_shared_prefix_equals_concatenated_keys(gpu, B, P, Sn, Sq, HK, splits, use_len):
     """mica_attention_fwd_prefix (a key prefix shared by every sequence, read in place) against the same
@@ -1145,6 +1158,7 @@ def test_attention_fused_rope_equals_rope_then_attention(gpu, B, P, S, HK, split
     (2, 64, 96, 128, "k", 200, True),       # a prefix continuation, k norm only, some positions off the table
     (1, 0, 70, 64, "", 50, False),          # partial RoPE alone
     (2, 0, 100, 0, "qk", 1, False),         # head norms alone
+    (2, 704, 96, 64, "qk", 4096, True),     # folded into the pipelined schedule, after a prefix
 ])
 def test_attention_fused_head_norm_rope_equals_passes(gpu, B, P, S, rot, norms, n_pos, use_pos):
     """mica_attention_fwd_rope with head norms and partial RoPE against head_norm_rope over the q and k
