@@ -6,13 +6,14 @@ and within one bf16 ulp where it is not (the fp32 summation order inside RMSNorm
 SiLU); option probabilities within 1e-3 absolute.  Shapes are the benchmark configurations; the
 largest ones are checked on a seeded sample of rows (rows of a GEMM are independent).
 """
+import ctypes
 import sys
 
 import numpy as np
 import pytest
 import torch
 
-from mica_amd import fused_kernels, int8_kernels, int8_runtime
+from mica_amd import _lib, fused_kernels, int8_kernels, int8_runtime
 from mica_amd.readout import LabelReadout
 from oracle import w8a8 as O
 
@@ -55,6 +56,15 @@ def assert_equal_diag(got, want, what):
     if bad.size:
         gv, wv = got.ravel()[bad[:6]], want.ravel()[bad[:6]]
         raise AssertionError(f"{what}: {bad.size} of {got.size} differ; at {bad[:6]} got {gv} want {wv}")
+
+
+def few_rows_tile(gpu, m, n, k, epi):
+    """(rows, weight rows, waves sharing K) of the small tiles a 16-bit-output GEMM runs on, None on another schedule."""
+    t = (ctypes.c_int * 3)()
+    cus = _lib.device_info(gpu.index)["cu_count"]
+    rc = _lib.load().mica_mm_i8_few_rows_tile(m, n, k, int8_kernels.EPILOGUE.get(epi, 0), cus, t)
+    assert rc >= 0
+    return tuple(t) if rc else None
 
 
 @pytest.fixture(autouse=True)
@@ -376,15 +386,22 @@ def test_gemm_extreme_accumulators(gpu):
     assert np.abs(acc).max() == k * 127 * 127
 
 
-@pytest.mark.parametrize("m", [1, 100, 128, 200, 300, 700])
-def test_gemm_silu_m_halves(gpu, m):
-    """The fused gate+up SiLU epilogue at N = 3072 runs as one round of 128 x 128 tiles (one gate / up
-    group each; rows past M in the last tile row), within one bf16 ulp of the oracle; with 32768 more
-    weight rows the same columns come from whole tiles and 128 x 256 halves along M (a lower half wholly
-    past M skipped, one cut by it, or both full), with the same bits."""
-    note(f"gemm silu m-halves m={m}")
+@pytest.mark.parametrize("m,n,k,small", [
+    (1, 3072, 2560, True), (100, 3072, 2560, True), (128, 3072, 2560, True), (200, 3072, 2560, True),
+    (300, 3072, 2560, True),
+    (385, 3072, 2560, False), (500, 3072, 2560, False), (700, 3072, 2560, False),
+    (129, 12288, 512, False), (100, 19456, 512, False),
+])
+def test_gemm_silu_m_halves(gpu, m, n, k, small):
+    """The fused gate+up SiLU epilogue in one round of 128 x 128 tiles (one gate / up group each; rows past M in the
+    last tile row), or of the smaller tiles of few rows, within one bf16 ulp of the oracle; with many more weight rows
+    the same columns come from whole tiles and 128 x 256 halves along M (a lower half wholly past M skipped, one cut
+    by it, or both full), with the same bits."""
+    note(f"gemm silu m-halves m={m} n={n} k={k}")
+    assert (few_rows_tile(gpu, m, n, k, "silu_mul") is not None) == small
+    more = 65536 if small and m <= 128 else 32768
+    assert few_rows_tile(gpu, m, n + more, k, "silu_mul") is None
     rng = np.random.default_rng(m + 5)
-    n, k = 3072, 2560
     A, B, sa, sb = _rand_gemm(rng, m, n, k)
     grp = B.reshape(n // 128, 2, 64, k)
     sgr = sb.reshape(n // 128, 2, 64)
@@ -392,13 +409,12 @@ def test_gemm_silu_m_halves(gpu, m):
     uv = O.epilogue(O.int_gemm(A, grp[:, 1].reshape(n // 2, k)), sa, sgr[:, 1].reshape(n // 2))
     y = int8_kernels.mm_i8(*(torch.from_numpy(v).cuda() for v in (A, sa, B, sb)), epilogue="silu_mul")
     assert_within_one_ulp(bits_of(y), O.silu_mul(gv, uv))
-    # here every M runs as one round of 128 x 128 tiles of one gate / up group each; with 32768 more
-    # weight rows (more 128 x 128 tiles than CUs: whole tiles, then M-halves or whole tiles for the tail)
-    # the same columns come out with the same bits: rows and column groups are independent
-    B2 = np.concatenate([B, rng.integers(-127, 128, (32768, k), dtype=np.int8)])
-    sb2 = np.concatenate([sb, rng.uniform(1e-3, 1e-2, 32768).astype(np.float32)])
+    # with that many more weight rows (more 128 x 128 tiles than CUs: whole tiles, then M-halves or whole tiles for
+    # the tail) the same columns come out with the same bits: rows and column groups are independent
+    B2 = np.concatenate([B, rng.integers(-127, 128, (more, k), dtype=np.int8)])
+    sb2 = np.concatenate([sb, rng.uniform(1e-3, 1e-2, more).astype(np.float32)])
     y2 = int8_kernels.mm_i8(*(torch.from_numpy(v).cuda() for v in (A, sa, B2, sb2)), epilogue="silu_mul")
-    assert np.array_equal(bits_of(y2)[:, : n // 2], bits_of(y)), "128 x 128 SiLU tiles differ from the other schedules"
+    assert np.array_equal(bits_of(y2)[:, : n // 2], bits_of(y)), "SiLU tiles of one round differ from the other schedules"
 
 
 def test_gemm_requant_output(gpu):
@@ -515,9 +531,10 @@ def test_gemm_headline_full_size(gpu):
 @pytest.mark.parametrize("m,n,k,epi", [
     (4096, 4352, 8192, "none"),      # 272 tiles: 256 whole, then 16 as 128 x 128 quarters (M > 256)
     (700, 2560, 9728, "residual"),   # 96 tiles of 128 x 160 leave room for 2 parts only: quarters
-    (300, 3072, 8192, "silu_mul"),   # 36 tiles of 128 x 256 in 3 parts along K, then the SiLU epilogue
+    (420, 3072, 8192, "silu_mul"),   # 48 tiles of 128 x 256 in 3 parts along K, then the SiLU epilogue
     (200, 2560, 8256, "none"),       # int32: 256 x 256 stream-K split, ranges straddle tiles; bf16: quarters
-    (256, 2560, 9728, "none"),       # 32 tiles of 128 x 160 in 3 parts (the int32 output: stream-K split)
+    (256, 2560, 9728, "none"),       # int32: 256 x 256 stream-K split; bf16: one round of small tiles, workspace unused
+    (448, 2560, 9728, "none"),       # bf16: 64 tiles of 128 x 160 in 3 parts; int32: quarters
     (512, 2560, 4096, "none"),       # K below both split thresholds: quarters, workspace unused
 ])
 def test_gemm_split_schedule_bit_exact(gpu, m, n, k, epi):
@@ -551,12 +568,13 @@ def test_gemm_split_schedule_bit_exact(gpu, m, n, k, epi):
 
 
 @pytest.mark.parametrize("m,n,k,epi", [
-    (128, 2560, 9728, "residual"),   # one short request's down projection: 16 tiles of 128 x 160, 3 parts
-    (128, 4096, 8192, "silu_mul"),   # SiLU epilogue: 16 tiles of 128 x 256, 3 parts of 21 or 22 slabs
-    (77, 6144, 8192, "none"),        # ragged M (51 empty rows in every tile), 39 tiles, 3 parts
+    # more rows, or more bytes a tile, than the small tiles of up to 384 rows serve
+    (385, 2560, 9728, "residual"),   # a request's down projection: 64 tiles of 128 x 160 (the last 1 row), 3 parts
+    (450, 2048, 8192, "silu_mul"),   # SiLU epilogue: 32 tiles of 128 x 256, 3 parts of 21 or 22 slabs
+    (500, 2568, 8192, "none"),       # ragged M and N, 68 tiles, 3 parts
     (512, 2560, 9728, "bias_fp16"),  # fp16 output with a bias, 64 tiles, 3 parts
-    (64, 2560, 16384, "none"),       # the most parts: 128 slabs in 6 parts, 16 tiles
-    (256, 2560, 8192, "bias_residual"),  # bias and residual together (bf16), 32 tiles, 3 parts
+    (200, 2048, 16384, "none"),      # the most parts: 128 slabs in 6 parts, 26 tiles
+    (400, 2560, 8192, "bias_residual"),  # bias and residual together (bf16), 64 tiles, 3 parts
 ])
 def test_gemm_small_m_split_bit_exact(gpu, m, n, k, epi):
     """Few 128-row tiles and a long K, with a workspace: every tile is split along K over several
@@ -564,6 +582,7 @@ def test_gemm_small_m_split_bit_exact(gpu, m, n, k, epi):
     so the output equals the unsplit schedule's bit for bit and the oracle's (the SiLU within the
     one-ulp bound of its own test), on two calls in a row (the arrival counts come back to zero)."""
     note(f"gemm small-M split m={m} n={n} k={k} epi={epi}")
+    assert few_rows_tile(gpu, m, n, k, epi) is None, "these sizes no longer reach the split along K"
     rng = np.random.default_rng(m + n + k + 7)
     A, B, sa, sb = _rand_gemm(rng, m, n, k)
     tA, tB, tsa, tsb = (torch.from_numpy(v).cuda() for v in (A, B, sa, sb))
@@ -610,33 +629,48 @@ def test_gemm_small_m_split_bit_exact(gpu, m, n, k, epi):
         assert np.array_equal(got.view(np.uint16), plain.view(np.uint16)), f"split != unsplit (call {rep})"
 
 
-@pytest.mark.parametrize("m,n,k,epi", [
-    (1, 2560, 9728, "residual"),        # 16 x 16 tiles, K split over 4 waves, 15 of 16 rows past the end
-    (17, 2568, 512, "bias"),            # 16 x 32, one slab, both edges ragged
-    (16, 10240, 2560, "none"),          # 16 x 64
-    (33, 2500, 1024, "bias_fp16"),      # 32 x 32, N a multiple of 4 only
-    (100, 2562, 4096, "residual"),      # 64 x 32, element stores (N even only)
-    (33, 9001, 512, "bias_residual"),   # 32 x 128, odd N
-    (384, 2560, 9728, "residual"),      # 64 x 64, K split over 2 waves, the most rows and bytes per tile
-    (200, 10240, 2560, "none"),         # 128 x 128
-    (127, 10240, 2560, "bias"),         # 128 x 64
-    (192, 10240, 2560, "none"),         # 64 x 128
-    (48, 300, 128, "none"),             # one slab of 128 bytes: the tiles that do not split K
-    (5, 32, 384, "none"),               # three slabs, N below a tile
-    (8, 19456, 2560, "silu_mul"),       # 32 x 128: 64 gate and 64 up rows
-    (64, 19456, 2560, "silu_mul"),      # 64 x 128
-    (128, 19456, 2560, "silu_mul"),     # 128 x 128
-    (20, 640, 512, "silu_mul"),         # 16 x 32: 16 gate and 16 up rows
-    (33, 3200, 1024, "silu_mul"),       # 32 x 32, ragged rows
-    (300, 4224, 256, "silu_mul"),       # 64 x 64, one slab, a last tile past the output
-    (131, 19456, 2048, "silu_mul"),     # 80 x 160, the second row tile 51 rows, 80 outputs a tile
-    (192, 19456, 2048, "silu_mul"),     # 96 x 192, the last tile 32 of 96 outputs wide
-    (300, 19456, 2560, "silu_mul"),     # 128 x 128 in two rounds
+@pytest.mark.parametrize("m,n,k,epi,tile", [
+    (1, 2560, 9728, "residual", (16, 16, 4)),       # 15 of a tile's 16 rows past the end
+    (5, 32, 512, "none", (16, 16, 4)),              # one slab, two tiles
+    (16, 6146, 512, "bias", (16, 32, 4)),           # the last tile 2 of 32 columns wide
+    (17, 2568, 512, "bias", (16, 32, 4)),           # both edges ragged
+    (16, 10240, 2560, "none", (16, 64, 4)),
+    (24, 6144, 2560, "bias_fp16", (32, 32, 4)),     # fp16
+    (33, 2500, 1024, "bias_fp16", (16, 32, 4)),     # N a multiple of 4 only
+    (24, 10240, 2560, "bias_residual", (32, 64, 4)),
+    (17, 9001, 512, "residual", (32, 64, 4)),       # odd N: element stores
+    (100, 2562, 4096, "residual", (64, 32, 4)),     # N even only
+    (33, 9001, 512, "bias_residual", (64, 64, 2)),
+    (384, 2560, 9728, "residual", (64, 64, 2)),     # the most rows and bytes per tile
+    (131, 6144, 2560, "none", (32, 128, 2)),        # an ordinary question's QKV, 3 rows in the last tile row
+    (5, 19460, 512, "bias_fp16", (32, 128, 2)),     # one row of tiles, the last 4 columns wide
+    (127, 10240, 2560, "bias", (128, 64, 1)),
+    (48, 300, 128, "none", (128, 64, 1)),           # one slab of 128 bytes: no wave shares K
+    (5, 32, 384, "none", (128, 64, 1)),             # three slabs, N below a tile
+    (192, 10240, 2560, "none", (64, 128, 1)),
+    (200, 10240, 2560, "none", (128, 128, 1)),
+    (300, 7170, 1536, "bias_residual", (128, 128, 1)),  # K at its line, ragged edges
+    (20, 640, 512, "silu_mul", (16, 32, 4)),        # 16 gate and 16 up rows
+    (9, 10240, 512, "silu_mul", (16, 64, 4)),
+    (20, 4224, 512, "silu_mul", (32, 32, 4)),
+    (33, 3200, 1024, "silu_mul", (32, 32, 4)),      # ragged rows
+    (20, 10240, 1024, "silu_mul", (32, 64, 4)),
+    (33, 4224, 512, "silu_mul", (64, 32, 4)),
+    (8, 19456, 2560, "silu_mul", (32, 128, 2)),     # 64 gate and 64 up rows
+    (40, 10240, 512, "silu_mul", (64, 64, 2)),
+    (300, 4224, 256, "silu_mul", (128, 64, 1)),     # two slabs, a last tile past the output
+    (64, 19456, 2560, "silu_mul", (64, 128, 1)),
+    (65, 19456, 2560, "silu_mul", (128, 128, 1)),
+    (128, 19456, 2560, "silu_mul", (80, 160, 1)),   # the second row tile 48 rows, the last tile 48 of 80 columns
+    (131, 19456, 2048, "silu_mul", (80, 160, 1)),
+    (192, 19456, 2048, "silu_mul", (96, 192, 1)),   # the last tile 32 of 96 columns wide
+    (300, 19456, 2560, "silu_mul", (128, 128, 1)),  # two rounds
 ])
-def test_gemm_few_rows_bit_exact(gpu, m, n, k, epi):
+def test_gemm_few_rows_bit_exact(gpu, m, n, k, epi, tile):
     """Up to 384 rows: one round of small tiles whose waves split K (int32 sums, exact in any order).  Bit-exact
     with the oracle; the SiLU within the one-ulp bound of its own test."""
     note(f"gemm few rows m={m} n={n} k={k} epi={epi}")
+    assert few_rows_tile(gpu, m, n, k, epi) == tile
     rng = np.random.default_rng(m * 5 + n + k)
     A, B, sa, sb = _rand_gemm(rng, m, n, k)
     tA, tB, tsa, tsb = (torch.from_numpy(v).cuda() for v in (A, B, sa, sb))
@@ -658,6 +692,41 @@ def test_gemm_few_rows_bit_exact(gpu, m, n, k, epi):
         rb = act_bits(rng, (m, n), outliers=0)
         res, ref = to_gpu_bf16(rb), O.f32_to_bf16(O.bf16_to_f32(ref) + O.bf16_to_f32(rb))
     assert_equal_diag(bits_of(int8_kernels.mm_i8(tA, tsa, tB, tsb, tb, residual=res)), ref, "bf16")
+
+
+@pytest.mark.parametrize("m,n,k,epi,tile", [
+    (17, 300, 512, "none", (16, 16, 4)),
+    (100, 2562, 1024, "none", (64, 32, 4)),
+    (33, 9001, 512, "none", (64, 64, 2)),
+    (70, 9000, 640, "none", (128, 64, 1)),
+    (257, 8002, 1536, "none", (128, 128, 1)),
+    (40, 4224, 512, "silu_mul", (64, 32, 4)),
+    (131, 19456, 2048, "silu_mul", (80, 160, 1)),
+])
+def test_gemm_few_rows_of_strided_operands(gpu, m, n, k, epi, tile):
+    """The C ABI's lda > K and ldb > K on the small tiles: the bits of contiguous operands, whatever the gaps hold;
+    the last row of each operand ends where its K elements do, and C's gaps keep what they had."""
+    note(f"gemm few rows strided m={m} n={n} k={k} epi={epi}")
+    assert few_rows_tile(gpu, m, n, k, epi) == tile
+    rng = np.random.default_rng(m + n + k)
+    tA, tB, tsa, tsb = (torch.from_numpy(v).cuda() for v in _rand_gemm(rng, m, n, k))
+    want = int8_kernels.mm_i8(tA, tsa, tB, tsb, epilogue=epi)
+    lda, ldb, n_out = k + 48, k + 144, n // 2 if epi == "silu_mul" else n
+    ldc = n_out + 7
+
+    def spaced(t, ld):
+        flat = torch.full(((t.shape[0] - 1) * ld + k,), 127, dtype=torch.int8, device=gpu)
+        flat.as_strided(t.shape, (ld, 1)).copy_(t)
+        return flat
+
+    wA, wB = spaced(tA, lda), spaced(tB, ldb)
+    out = torch.full((m, ldc), 3.0, dtype=torch.bfloat16, device=gpu)
+    rc = _lib.load().mica_mm_i8(wA.data_ptr(), lda, wB.data_ptr(), ldb, tsa.data_ptr(), tsb.data_ptr(), None, None, 0,
+                                out.data_ptr(), ldc, _lib.BF16, m, n, k, int8_kernels.EPILOGUE[epi], None, 0,
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(out[:, :n_out].contiguous().view(torch.int16), want.view(torch.int16))
+    assert (out[:, n_out:] == 3.0).all()
 
 
 @pytest.mark.parametrize("m,n,k", [(32768, 6144, 2560), (32768, 2560, 4096)])
@@ -1038,7 +1107,6 @@ def test_attention_split_keys_matches_oracle(gpu, B, Sq, Sk, HK, splits):
 def test_attention_schedules_agree_bit_for_bit(gpu, B, S, P, Sq):
     """Few workgroups over long keys run the pipelined schedule, more of them the other: the sequences of a batch run
     together and alone must agree in every bit (the same arithmetic per query)."""
-    from mica_amd import _lib
     from mica_amd.attention import causal_gqa_attention
 
     note(f"attention schedules B={B} S={S} P={P} Sq={Sq}")

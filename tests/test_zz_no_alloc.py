@@ -71,10 +71,12 @@ def test_scratch_size_is_stated(gpu):
 
 @pytest.mark.parametrize("calls", [
     # (m, n, k, epilogue) per call; the second call of each pair is smaller
-    # split rounds of 10 then 5 tiles of 256 x 256 (int32), 32 then 8 of 128 x 160 in 3 parts (bf16)
+    # split rounds of 10 then 5 tiles of 256 x 256 (int32); bf16: one round of small tiles, scratch unused
     ((256, 2560, 9728, "scale"), (128, 1280, 8192, "scale")),
-    # SiLU epilogue: 16 then 4 tiles of 128 x 256 in 3 parts
-    ((200, 2048, 8192, "silu_mul"), (64, 1024, 8192, "silu_mul")),
+    # bf16: 64 then 32 tiles of 128 x 160 in 3 parts (int32: quarter tiles)
+    ((500, 2560, 9728, "scale"), (400, 1280, 8192, "scale")),
+    # SiLU epilogue: 32 then 16 tiles of 128 x 256 in 3 parts
+    ((450, 2048, 8192, "silu_mul"), (390, 1024, 8192, "silu_mul")),
     # no split (K below both thresholds): quarter / half tiles
     ((512, 2560, 4096, "scale"), (300, 1000, 2576, "scale")),
 ])
@@ -119,19 +121,21 @@ def _capture_child():
     dev = torch.device("cuda", 0)
     L = _lib.load()
     rng = np.random.default_rng(21)
-    m, n, k = 256, 2560, 9728                    # split: 10 tiles of 256 x 256 (int32), 32 of 128 x 160 (bf16)
+    m, n, k = 256, 2560, 9728                    # split: 10 tiles of 256 x 256 (int32)
+    mh = 448                                     # and 64 of 128 x 160 (bf16)
     A, B, sa, sb = _operands(rng, m, n, k, dev)
+    Ah, _, sah, _ = _operands(rng, mh, n, k, dev)
     eager_i32 = torch.empty((m, n), dtype=torch.int32, device=dev)
-    eager_bf16 = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    eager_bf16 = torch.empty((mh, n), dtype=torch.bfloat16, device=dev)
     assert _call(False, A, B, sa, sb, eager_i32, _lib.INT32, _lib.EPI_SCALE) == 0
-    assert _call(False, A, B, sa, sb, eager_bf16, _lib.BF16, _lib.EPI_SCALE) == 0
+    assert _call(False, Ah, B, sah, sb, eager_bf16, _lib.BF16, _lib.EPI_SCALE) == 0
     out_i32 = torch.full((m, n), -1, dtype=torch.int32, device=dev)
-    out_bf16 = torch.full((m, n), -1, dtype=torch.bfloat16, device=dev)
+    out_bf16 = torch.full((mh, n), -1, dtype=torch.bfloat16, device=dev)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         rc = [_call(True, A, B, sa, sb, out_i32, _lib.INT32, _lib.EPI_SCALE),
-              _call(True, A, B, sa, sb, out_bf16, _lib.BF16, _lib.EPI_SCALE)]
+              _call(True, Ah, B, sah, sb, out_bf16, _lib.BF16, _lib.EPI_SCALE)]
     result = {"rc": rc, "replays": []}
     rows = np.unique(np.r_[0, m - 1, rng.integers(0, m, 6)])
     want = O.int_gemm(A.cpu().numpy()[rows], B.cpu().numpy())
@@ -152,7 +156,7 @@ def _capture_child():
 
 def test_noalloc_first_call_under_graph_capture(gpu):
     """A caller under HIP-graph capture whose first noalloc call is the captured one (see _capture_child)."""
-    note("noalloc first call inside graph capture: m=256 n=2560 k=9728, child process")
+    note("noalloc first call inside graph capture: m=256 and 448, n=2560 k=9728, child process")
     here = Path(__file__).resolve().parent
     code = f"import sys; sys.path[:0] = [{str(here.parent)!r}, {str(here)!r}]; import test_zz_no_alloc as t; t._capture_child()"
     proc = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=240,
