@@ -305,11 +305,14 @@ __global__ __launch_bounds__(kFaThreads, PIPE ? 1 : 2) void fa_fwd_kernel(FaPara
                                                      ln * 16, jj * kVBytes + (wave * 4 + i) * 1024, 0, 0);
     };
 
-    // The pipelined schedule's DMA, an instruction range at a time (addresses and sizes as scalars; a tile's resource is
-    // built where it is used).
-    const uint64_t ka = (uint64_t)(p.k + b * p.sbk + hk * p.shk), va = (uint64_t)(p.vt + ((long long)(b * p.HK + hk) * ntn) * kD * kBK);
-    const uint64_t kpa = (uint64_t)(ntp ? p.kp + hk * p.shkp : p.k), vpa = (uint64_t)(ntp ? p.vtp + ((long long)hk * ntp) * kD * kBK : p.vt);
-    const int kn = (int)((long long)(p.Sk - pk) * p.ldk * 2), vn = ntn * kVBytes, kpn = (int)((long long)pk * p.ldkp * 2), vpn = ntp * kVBytes;
+    // The pipelined schedule's DMA, an instruction range at a time (addresses and sizes as scalars; a tile's
+    // resource is built where it is used).
+    const uint64_t ka = (uint64_t)(p.k + b * p.sbk + hk * p.shk);
+    const uint64_t va = (uint64_t)(p.vt + ((long long)(b * p.HK + hk) * ntn) * kD * kBK);
+    const uint64_t kpa = (uint64_t)(ntp ? p.kp + hk * p.shkp : p.k);
+    const uint64_t vpa = (uint64_t)(ntp ? p.vtp + ((long long)hk * ntp) * kD * kBK : p.vt);
+    const int kn = (int)((long long)(p.Sk - pk) * p.ldk * 2), kpn = (int)((long long)pk * p.ldkp * 2);
+    const int vn = ntn * kVBytes, vpn = ntp * kVBytes;
     int8_t *const sm = smem;
     int ko_own[4], ko_diff[4]; // a prefix tile's offset less an own tile's
     const int tile_own = (int)(kBK * p.ldk * 2), tile_pre = (int)(kBK * p.ldkp * 2);
@@ -323,8 +326,8 @@ __global__ __launch_bounds__(kFaThreads, PIPE ? 1 : 2) void fa_fwd_kernel(FaPara
     // the same number of vector memory operations (which its vmcnt waits count).
     auto dma_k = [=](int j, int st, int i0, int i1) {
         const bool pre = j < ntp;  // the tile's segment: the shared prefix or this sequence's own keys
-        const uint64_t at = pre ? kpa + 0 : ka + 0;
-        const int n = j > last_own ? 0 : pre ? kpn + 0 : kn + 0, tile_off = pre ? j * tile_pre : (j - ntp) * tile_own;
+        const uint64_t at = pre ? kpa : ka;
+        const int n = j > last_own ? 0 : pre ? kpn : kn, tile_off = pre ? j * tile_pre : (j - ntp) * tile_own;
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)at, 0, n, kBufferFlags);
 #pragma unroll
         for (int i = i0; i < i1; ++i)
@@ -333,13 +336,14 @@ __global__ __launch_bounds__(kFaThreads, PIPE ? 1 : 2) void fa_fwd_kernel(FaPara
     };
     auto dma_v = [=](int j, int st, int i0, int i1) {
         const bool pre = j < ntp;
-        const uint64_t at = pre ? vpa + 0 : va + 0;
-        const int n = j > last_own || j < first ? 0 : pre ? vpn + 0 : vn + 0, jj = pre ? j : j - ntp;
+        const uint64_t at = pre ? vpa : va;
+        const int n = j > last_own || j < first ? 0 : pre ? vpn : vn, jj = pre ? j : j - ntp;
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)at, 0, n, kBufferFlags);
 #pragma unroll
         for (int i = i0; i < i1; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(sm + kPSt * kKBytes + st * kVBytes + (wave * 4 + i) * 1024),
-                                                     16, lane * 16, jj * kVBytes + (wave * 4 + i) * 1024, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                r, (lds_void *)(sm + kPSt * kKBytes + st * kVBytes + (wave * 4 + i) * 1024), 16, lane * 16,
+                jj * kVBytes + (wave * 4 + i) * 1024, 0, 0);
     };
 
     // Q fragments (B operand of S^T): lane holds query q0 + l % 32, dims 16 s + 8 (l / 32) .. + 7
