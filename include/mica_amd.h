@@ -124,9 +124,10 @@ int mica_rmsnorm_quant_multi(const void *x, int x_dtype, int ldx, const void *re
  * 16-byte aligned, whose first 4 KiB are zero before its first use (every launch leaves them zero
  * again).  With it, two schedules split tiles along K:
  *   - 16-bit outputs (SILU_MUL included), K % 256 == 0, K >= 8192: when the output fits at most CUs / 3
- *     tiles of 128 x 160 (SCALE) or 128 x 256 (SILU_MUL) -- a short request's down projection, e.g.
- *     M <= 512 at N = 2560 -- every tile is split into K / 2560 parts (at least 3), one workgroup per
- *     part, and each tile's last part adds the others' partial sums;
+ *     tiles of 128 x 160 (SCALE) or 128 x 256 (SILU_MUL) and no small tile covers it in one round
+ *     (mica_mm_i8_few_rows_tile) -- e.g. 385 to 512 rows of a down projection to N = 2560 -- every tile is
+ *     split into K / 2560 parts (at least 3), one workgroup per part, and each tile's last part adds the
+ *     others' partial sums;
  *   - int32 / fp32 outputs: when the last round of 256 x 256 tiles would hold at most CUs / 4 tiles,
  *     K >= 8192 and M <= 256 (elsewhere 128 x 128 quarter tiles, which need no workspace, serve such
  *     a round better), those tiles are split along K over four workgroups each.
@@ -142,9 +143,10 @@ int mica_mm_i8(const int8_t *A, int lda, const int8_t *B, int ldb, const float *
 /* bytes of GEMM workspace for `device` (its CU count x 512 KiB + 4 KiB), or -(hipError_t) */
 long long mica_mm_i8_workspace_bytes(int device);
 
-/* 1 when a 16-bit-output mica_mm_i8 of these sizes on a device of `cus` compute units runs as one round of small tiles
- * (no workspace needed), tile[0 .. 2] then being the tile's rows, its weight rows and the waves that share K; 0 when
- * another schedule runs, -1 for invalid sizes.  (Operands that reach 2^31 bytes a tile past their last row never do.) */
+/* 1 when a 16-bit-output mica_mm_i8 of these sizes runs, on a device of `cus` compute units, on the small tiles of few
+ * rows (no workspace needed), tile[0 .. 2] then being the tile's rows, its weight rows and the waves that share K; 0
+ * when another schedule runs, -1 for invalid sizes.  (Operands that reach 2^31 bytes a tile past their last row never
+ * run on them.) */
 int mica_mm_i8_few_rows_tile(int M, int N, int K, int epilogue, int cus, int *tile);
 
 /*
@@ -317,7 +319,8 @@ int mica_attention_fwd_prefix(const void *q, long long sbq, long long shq, long 
 long long mica_attention_prefix_workspace_bytes(int B, int Sq, int Sk, int Pk, int HQ, int HK, int key_splits);
 
 /* 1 when an unsplit attention launch of these sizes (any entry point; Sk counts a prefix's keys) runs the pipelined
- * schedule on a device of `cus` compute units, 0 when two workgroups per CU, -1 for invalid sizes; same bits either way */
+ * schedule on a device of `cus` compute units, 0 when the one with two workgroups per CU, -1 for invalid sizes; the
+ * bits are the same */
 int mica_attention_pipelined(int B, int Sq, int Sk, int HK, int cus);
 
 /*

@@ -84,8 +84,8 @@ using QNarrow = QCfg<256, 160, 2, 4, 1>;
 // 256 x 256 tiles lost by it (4096 x 9728 x 2560 86.5 -> 91.7 us, 4096 x 6144 x 2560 57.3 -> 58.6, the
 // 256 x 160 tiles of 4096 x 2560 x 9728 79.0 -> 80.0; interleaved on one box).
 using QSmall = QCfg<128, 160, 4, 4, 1, 2>;
-// The SiLU epilogue's counterpart for launches of at most 128 rows that gemm_i8_thin.hip has no tile for
-// (K not a multiple of 128, 73 and more rows with K < 2048): one round
+// The SiLU epilogue's counterpart (K a multiple of 256, at least 512) wherever its 128 x 128 tiles fit one round
+// and gemm_i8_thin.hip takes no tile (more than 384 rows, or its rule leaves the launch here): one round
 // of 128 x 128 tiles, each one 64-row group of gate weights and its 64 up rows, on waves of 32 x 128
 // stacked along M (2 x 8 MFMA tiles, 64 accumulators per lane), so every wave pairs gate and up columns
 // in its own lanes.  128 x 19456 x 2560: 152 tiles on 152 CUs, where the 128 x 256 M-halves keep 76

@@ -6,9 +6,10 @@
 // 128-row and larger tiles of the other kernels leave most CUs idle there (128 x 2560 x 9728: 16 tiles of
 // 128 x 160).  So tiles are as small as one round allows (thin_pick), and where such a tile has fewer fragments
 // than waves, WK of the 4 to 8 waves take their own 128 bytes of every slab and the int32 partial sums meet in LDS at
-// the end (exact in any order: same bits as every other schedule; no workspace, no second workgroup).  NS slabs
-// are in flight per workgroup, up to 144 KiB.
-// Measured on MI355X, weights cold in the caches (24 copies in turn), us, before -> this kernel:
+// the end (exact in any order: same bits as every other schedule; no workspace, no second workgroup).  NS stages
+// of LDS hold the slabs in flight, up to 150 KiB per workgroup.
+// Measured on MI355X, weights cold in the caches (24 copies in turn), us, what QLinear ran before (K = 9728: split
+// along K) -> this kernel:
 //   M x N x K                8 rows         64 rows        128 rows       256 rows
 //   2560 x 9728 + residual   21.2 ->  8.2   24.0 -> 14.0   27.0 -> 19.0   27.4 -> 24.4
 //   2560 x 4096 + residual   13.0 ->  4.4   13.3 ->  5.7   14.2 ->  7.4   14.4 ->  9.3
